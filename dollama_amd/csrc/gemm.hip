@@ -571,10 +571,10 @@ __device__ __forceinline__ i32x4 dma_rsrc(const void* p, unsigned bytes) {
 // drains it: the kernel orders it with explicit vmcnt waits and barriers.
 // Nothing else in this file uses M0, so clobbering it is safe although the
 // compiler warns that it treats M0 as reserved.
-__device__ __forceinline__ void dma16(const i32x4& r, const unsigned char DLM_LDS* dst, int voff) {
+__device__ __forceinline__ void dma16(const i32x4& r, const unsigned char DLM_LDS* dst, int voff, int soff) {
   const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds),
-               "v"(voff), "s"(r)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
+               "v"(voff), "s"(r), "s"(soff)
                : "memory", "m0");
 }
 
@@ -593,124 +593,173 @@ __device__ __forceinline__ int dma_row(int nw, int i, int wave, int lane) {
 }
 __device__ __forceinline__ int dma_chunk(int row, int lane) { return (lane & 7) ^ ((row >> 1) & 7); }
 
+// Both loaders hand the DMA a per-lane offset voff[i] that rarely changes
+// (the lane's row and chunk) and a wave-uniform offset soff that moves with
+// the K slice, so a slice costs a few scalar instructions instead of a
+// recomputed address per lane.
 template <int I>
 struct RowDma {
   i32x4 rs;
-  int base[I];  // byte offset of the lane's chunk in K-slice 0, -1 past the last row
-  int kc[I];    // K index of that chunk within a slice
+  int voff[I];  // byte offset of the lane's chunk in K-slice 0, kOOB past the last row
+  int soff;
+  int kc;       // K index of the lane's first chunk within a slice
   int K;
   __device__ RowDma(const RowDesc& d, int r0, int nw, int wave, int lane)
-      : rs(dma_rsrc(d.p, d.bytes)), K(d.K) {
+      : rs(dma_rsrc(d.p, d.bytes)), soff(0), K(d.K) {
 #pragma unroll
     for (int i = 0; i < I; ++i) {
       const int row = dma_row(nw, i, wave, lane);
-      const int c = dma_chunk(row, lane);
-      kc[i] = c * 8;
-      base[i] = r0 + row < d.rows ? ((r0 + row) * d.ld + c * 8) * 2 : -1;
+      voff[i] = r0 + row < d.rows ? ((r0 + row) * d.ld + dma_chunk(row, lane) * 8) * 2 : kOOB;
     }
+    // nw * 8 rows between a wave's DMA instructions: a multiple of 16, so
+    // every instruction of the lane covers the same chunk
+    kc = dma_chunk(dma_row(nw, 0, wave, lane), lane) * 8;
   }
   __device__ __forceinline__ void seek(int) {}
-  __device__ __forceinline__ void prepare(int) {}
-  __device__ __forceinline__ int off(int i, int kt) const {
-    return (base[i] >= 0 && kt * BK + kc[i] < K) ? base[i] + kt * (BK * 2) : kOOB;
+  __device__ __forceinline__ void prepare(int kt) {
+    soff = kt * (BK * 2);
+    if (kt * BK + BK > K) {  // uniform: the last slice of a K that is no multiple of 64
+#pragma unroll
+      for (int i = 0; i < I; ++i) voff[i] = kt * BK + kc < K ? voff[i] : kOOB;
+    }
   }
 };
 
 // Implicit-im2col rows for the DMA path (C0, C0a, C1, C1a multiples of 64:
-// one tap and one source per K slice, both wave-uniform).  Every parameter is
-// copied into registers (the DMA asm clobbers memory, which would otherwise
-// force kernel-argument reloads inside the loop) and the per-lane offset is
-// computed with selects only.
+// one tap and one source per K slice, both wave-uniform).
+//
+// The K order is: 64-channel blocks of source 0a, then of 0b, each with its
+// KH*KW taps inside (so the slices that re-read one block of a pixel's
+// channels run back to back and find its lines in the L2), then the blocks of
+// the 1x1 sources 1a and 1b.  A slice's position is tap (kh, kw) of block c.
+//
+// The lane's offset is that of tap (0, 0), plus `inv`, one bit per kh (0-15)
+// and per kw (16-31) that is set where the tap falls outside the image: three
+// VALU instructions put the tap's two bits into the offset's sign bit, which
+// the buffer range check turns into zeros.  The tap's own displacement is
+// uniform and goes into soff.  A tap (0, 0) may lie before the image, so the
+// descriptor starts that many bytes early and every offset is raised by as
+// much (valid lanes never reach the raised part).  Recomputing the pixel and
+// its bounds per lane and slice made the loader the longest part of a slice's
+// issue (about 64 VALU and 100 scalar instructions of a 256x160 tile's 240):
+// 3x3 conv 2x128x128x320 69.4 -> 62.6 us, VAE decode 18.4 -> 17.0 ms.  Nearest-2x upsampling
+// halves the tap's coordinate, ((p + kh) >> 1) = (kh >> 1) + (p & kh & 1) for
+// a lane of parity p: a uniform part and one masked add per axis.
 __device__ __forceinline__ int rfl(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 template <int I>
 struct ConvDma {
-  int pbase[I], ihb[I], iwb[I], mrow[I], cch[I];
-  // uniform parameters
-  const f16 *s0a, *s0b, *s1a, *s1b;
-  unsigned bytes0a, bytes0b, bytes1a, bytes1b;
-  int C0, C0a, ld0a, ld0b, C1, C1a, ld1a, ld1b, K0, KH, KW, Hv, Wv, W, up, M, dil_h, dil_w;
-  // per-slice state
+  const ConvParams& d;
   i32x4 rs;
-  int seg, kh, kw, ld, cbase;
-  __device__ ConvDma(const ConvParams& d, int m0, int nw, int wave, int lane)
-      : s0a(d.s0a), s0b(d.s0b), s1a(d.s1a), s1b(d.s1b), bytes0a(d.bytes0a), bytes0b(d.bytes0b),
-        bytes1a(d.bytes1a), bytes1b(d.bytes1b), C0(d.C0), C0a(d.C0a), ld0a(d.ld0a), ld0b(d.ld0b),
-        C1(d.C1), C1a(d.C1a), ld1a(d.ld1a), ld1b(d.ld1b), K0(d.K0), KH(d.KH), KW(d.KW), Hv(d.Hv), Wv(d.Wv),
-        W(d.W), up(d.up), M(d.M), dil_h(d.dil_h), dil_w(d.dil_w) {
+  int voff[I];
+  int soff;
+  int base[I], inv[I];
+  int m0, nw, wave, lane;
+  int seg;                     // 0 / 1: source 0a / 0b, 2 / 3: source 1a / 1b
+  int KH, KW;                  // taps of the segment
+  int row_step, col_step;      // bytes per kh / kw step (upsampling: per stored row / pixel)
+  int up;
+  int cur_kt, kh, kw, c, cend;  // c, cend: byte offset of the channel block, end of the segment
+  __device__ ConvDma(const ConvParams& dd, int m0_, int nw_, int wave_, int lane_)
+      : d(dd), m0(m0_), nw(nw_), wave(wave_), lane(lane_) {}
+  __device__ __forceinline__ void segment(int sg, int blk) {
+    seg = sg;
+    const bool second = sg & 1;
+    cur_kt = -1;
+    if (sg < 2) {
+      const int ld = second ? d.ld0b : d.ld0a;
+      const int shift = d.pad_h * d.W + d.pad_w;  // pixels before the image
+      rs = dma_rsrc((second ? d.s0b : d.s0a) - (size_t)shift * ld, 0x80000000u);
+      KH = rfl(d.KH);
+      KW = rfl(d.KW);
+      up = rfl(d.up);
+      row_step = rfl(d.dil_h * d.W * ld * 2);
+      col_step = rfl(d.dil_w * ld * 2);
+      c = rfl(blk * (BK * 2));
+      cend = rfl((second ? d.C0 - d.C0a : d.C0a) * 2);
 #pragma unroll
-    for (int i = 0; i < I; ++i) {
-      const int row = dma_row(nw, i, wave, lane);
-      cch[i] = dma_chunk(row, lane) * 8;
-      const int m = m0 + row;
-      mrow[i] = m;
-      const int mm = m < d.M ? m : 0;
-      const int n = mm / d.HoWo;
-      const int q = mm - n * d.HoWo;
-      const int oh = q / d.Wo;
-      const int ow = q - oh * d.Wo;
-      pbase[i] = m < d.M ? n * d.H * d.W : -1;
-      ihb[i] = oh * d.stride_h - d.pad_h;
-      iwb[i] = ow * d.stride_w - d.pad_w;
+      for (int i = 0; i < I; ++i) {
+        const int row = dma_row(nw, i, wave, lane);
+        const int m = m0 + row;
+        const int mm = m < d.M ? m : 0;
+        const int n = mm / d.HoWo;
+        const int q = mm - n * d.HoWo;
+        const int oh = q / d.Wo;
+        const int ihb = oh * d.stride_h - d.pad_h, iwb = (q - oh * d.Wo) * d.stride_w - d.pad_w;
+        const int pix = (n * d.H + (ihb >> up)) * d.W + (iwb >> up) + shift;
+        base[i] = (pix * ld + dma_chunk(row, lane) * 8) * 2;
+        unsigned bits = 0;
+        for (int t = 0; t < d.KH; ++t) bits |= (unsigned)((unsigned)(ihb + t * d.dil_h) >= (unsigned)d.Hv) << t;
+        for (int t = 0; t < d.KW; ++t)
+          bits |= (unsigned)((unsigned)(iwb + t * d.dil_w) >= (unsigned)d.Wv) << (16 + t);
+        bits |= up ? (unsigned)(ihb & 1) << 14 | (unsigned)(iwb & 1) << 30 : 0u;
+        inv[i] = m < d.M ? (int)bits : -1;
+      }
+    } else {
+      const int ld = second ? d.ld1b : d.ld1a;
+      rs = dma_rsrc(second ? d.s1b : d.s1a, second ? d.bytes1b : d.bytes1a);
+      KH = KW = 1;
+      up = 0;
+      row_step = col_step = 0;
+      c = rfl(blk * (BK * 2));
+      cend = rfl((second ? d.C1 - d.C1a : d.C1a) * 2);
+#pragma unroll
+      for (int i = 0; i < I; ++i) {
+        const int row = dma_row(nw, i, wave, lane);
+        const int m = m0 + row;
+        base[i] = (m * ld + dma_chunk(row, lane) * 8) * 2;
+        inv[i] = m < d.M ? 0 : -1;
+      }
+    }
+    kh = kw = 0;
+  }
+  // position at slice kt (start of the range)
+  __device__ __forceinline__ void seek(int kt) {
+    const int taps = d.KH * d.KW;
+    const int cb = kt / taps, nb0 = d.C0 / BK, na0 = d.C0a / BK, na1 = d.C1a / BK;
+    const bool s0 = cb < nb0;
+    const int k1 = kt - nb0 * taps;
+    const bool second = s0 ? cb >= na0 : k1 >= na1;
+    segment((s0 ? 0 : 2) + (int)second, s0 ? cb - (second ? na0 : 0) : k1 - (second ? na1 : 0));
+    const int tap = s0 ? kt - cb * taps : 0;
+    kh = rfl(tap / d.KW);
+    kw = rfl(tap - kh * d.KW);
+    cur_kt = kt;
+    place();
+  }
+  __device__ __forceinline__ void place() {
+    const int rr = up ? kh >> 1 : kh, cc = up ? kw >> 1 : kw;
+    soff = rfl(rr * row_step + cc * col_step + c);
+    const int sh = 31 - kh, sw = 15 - kw;
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+      voff[i] = (int)((((unsigned)inv[i] << sh) | ((unsigned)inv[i] << sw)) & 0x80000000u) | base[i];
+    if (up) {  // uniform; bits 14 and 30 of inv: the parity of the row and of the column
+      const int rs_ = (kh & 1) ? row_step : 0, cs_ = (kw & 1) ? col_step : 0;
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+        voff[i] += (__builtin_amdgcn_sbfe(inv[i], 14, 1) & rs_) + (__builtin_amdgcn_sbfe(inv[i], 30, 1) & cs_);
     }
   }
-  // Segment-0 K order: 64-channel blocks outermost, then the taps (kh, kw),
-  // so the KH*KW slices that re-read one block of a pixel's channels run
-  // back to back and find its lines still in the L2.  Slices are requested
-  // in order (kb, kb+1, ..., then the last one repeated), so the tap /
-  // channel position advances by one slice at a time: no integer division
-  // and no branch in the loop (all selects).
-  int cur_kt = 0, cur_c = 0, cur_kh = 0, cur_kw = 0;
-  // position the tap state at slice kt (start of a split-K range)
-  __device__ __forceinline__ void seek(int kt) {
-    const int taps = KH * KW;
-    const bool s0 = kt * BK < K0;
-    const int cb = s0 ? kt / taps : 0;
-    const int tap = s0 ? kt - cb * taps : 0;
-    cur_kt = kt;
-    cur_c = rfl(cb * BK);
-    cur_kh = rfl(tap / KW);
-    cur_kw = rfl(tap - (tap / KW) * KW);
-  }
+  // Slices are requested in order (kb, kb+1, ..., then the last one repeated)
   __device__ __forceinline__ void prepare(int kt) {
-    const bool adv = kt != cur_kt;  // kt == cur_kt + 1
-    int kw1 = cur_kw + 1;
-    const bool wrapw = kw1 == KW;
-    kw1 = wrapw ? 0 : kw1;
-    int kh1 = cur_kh + (wrapw ? 1 : 0);
-    const bool wraph = kh1 == KH;
-    kh1 = wraph ? 0 : kh1;
-    const int c1 = cur_c + (wraph ? BK : 0);
-    cur_c = rfl(adv ? c1 : cur_c);
-    cur_kw = rfl(adv ? kw1 : cur_kw);
-    cur_kh = rfl(adv ? kh1 : cur_kh);
+    if (kt == cur_kt) return;
     cur_kt = kt;
-    const int k0 = kt * BK;
-    const bool s1 = k0 >= K0;
-    const int cs = k0 - K0;  // segment-1 K index of the slice
-    const bool isa0 = cur_c < C0a, isa1 = cs < C1a;
-    // arithmetic selects throughout: a ternary between members lets the
-    // compiler select their addresses instead, which moves them to scratch
-    const f16* src = pick(s1, pick(isa1, s1a, s1b), pick(isa0, s0a, s0b));
-    const unsigned bytes = pick(s1, pick(isa1, bytes1a, bytes1b), pick(isa0, bytes0a, bytes0b));
-    rs = dma_rsrc(src, bytes);
-    ld = rfl(pick(s1, pick(isa1, ld1a, ld1b), pick(isa0, ld0a, ld0b)));
-    cbase = rfl(pick(s1, pick(isa1, cs, cs - C1a), pick(isa0, cur_c, cur_c - C0a)));
-    kh = rfl(pick(s1, cs, cur_kh * dil_h));  // segment 0: tap offset in input rows
-    kw = rfl(pick(s1, 0, cur_kw * dil_w));
-    seg = rfl(s1 ? 1 : 0);
-  }
-  // Both segment offsets are always computed and chosen with arithmetic
-  // selects, so the DMA sequence stays free of divergent branches.
-  __device__ __forceinline__ int off(int i, int) const {
-    int ih = ihb[i] + kh, iw = iwb[i] + kw;
-    const bool ok0 = (pbase[i] >= 0) & ((unsigned)ih < (unsigned)Hv) & ((unsigned)iw < (unsigned)Wv);
-    ih >>= up;
-    iw >>= up;
-    const int o0 = ((pbase[i] + ih * W + iw) * ld + cbase + cch[i]) * 2;
-    const bool ok1 = (mrow[i] < M) & (kh + cch[i] < C1);
-    const int o1 = (mrow[i] * ld + cbase + cch[i]) * 2;
-    return pick(seg == 0, pick(ok0, o0, kOOB), pick(ok1, o1, kOOB));
+    const bool wrapw = kw + 1 == KW;
+    kw = rfl(wrapw ? 0 : kw + 1);
+    const int kh1 = kh + (wrapw ? 1 : 0);
+    const bool wraph = kh1 == KH;
+    kh = rfl(wraph ? 0 : kh1);
+    c = rfl(c + (wraph ? BK * 2 : 0));
+    if (c == cend) {  // uniform, at most three times a tile: the next source that has channels
+      const int k = cur_kt;
+      int sg = seg + 1;
+      if (sg == 1 && d.C0 == d.C0a) sg = 2;
+      if (sg == 2 && d.C1a == 0) sg = 3;
+      segment(sg, 0);
+      cur_kt = k;
+    }
+    place();
   }
 };
 
@@ -1152,15 +1201,16 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
   // past the last row group)
   auto dma_a = [&](unsigned char DLM_LDS* st, int i, int kt) {
     if (IA * NW == GA || i + 1 < IA || wave < GA - (IA - 1) * NW)
-      dma16(al.rs, st + (i * NW + wave) * 1024, al.off(i, kt));
+      dma16(al.rs, st + (i * NW + wave) * 1024, al.voff[i], al.soff);
   };
   auto dma_b = [&](unsigned char DLM_LDS* st, int i, int kt) {
     if (IB * NW == GB || i + 1 < IB || wave < GB - (IB - 1) * NW)
-      dma16(bl.rs, st + SA + (i * NW + wave) * 1024, bl.off(i, kt));
+      dma16(bl.rs, st + SA + (i * NW + wave) * 1024, bl.voff[i], bl.soff);
   };
   auto issue_all = [&](int buf, int kt) {
     unsigned char DLM_LDS* st = smem + buf * STAGE;
     al.prepare(kt);
+    bl.prepare(kt);
 #pragma unroll
     for (int i = 0; i < IA; ++i) dma_a(st, i, kt);
 #pragma unroll
@@ -1216,6 +1266,7 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
         unsigned char DLM_LDS* dst = smem + t * STAGE + j * SLICE;
         const int kt = slice_kt(t, j);
         al.prepare(kt);
+        bl.prepare(kt);
 #pragma unroll
         for (int i = 0; i < IA; ++i) dma_a(dst, i, kt);
 #pragma unroll
@@ -1266,6 +1317,7 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
           const int r = q >> 1;
           const int kt = slice_kt(t + NS - 1, r);
           al.prepare(kt);
+          bl.prepare(kt);
 #pragma unroll
           for (int i = 0; i < IA; ++i) dma_a(nst + r * SLICE, i, kt);
         } else {
@@ -1346,6 +1398,7 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
     unsigned char DLM_LDS* nst = smem + pnslot * STAGE;
     const int nkt = min(kt + NS - 1, ke - 1);
     al.prepare(nkt);
+    bl.prepare(nkt);
     f16x8 fa[2][TM], fb[2][TN];
     auto rd = [&](int ks) {
 #pragma unroll
@@ -1728,7 +1781,11 @@ static bool dma_epilogue_ok(const EpiArgs& ep) {
 }
 static bool dma_operand_ok(const RowDesc& a) { return dlm_aligned16(a.p) && a.ld % 8 == 0; }
 static bool dma_operand_ok(const ConvDesc& d) {
-  return !d.generic && d.C1 % BK == 0 && d.C1a % BK == 0;
+  // ConvDma packs a lane's tap validity into 14 + 14 bits and raises its
+  // offsets by the padding in front of the image plus a row and a pixel
+  const unsigned long long raise = ((unsigned long long)(d.pad_h + 1) * d.W + d.pad_w + 1) * 2;
+  return !d.generic && d.C1 % BK == 0 && d.C1a % BK == 0 && d.KH <= 14 && d.KW <= 14 &&
+         std::max(d.bytes0a + raise * d.ld0a, d.bytes0b + raise * d.ld0b) < (1ull << 31);
 }
 
 template <class Desc>
