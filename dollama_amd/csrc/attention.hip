@@ -276,7 +276,6 @@ __device__ __forceinline__ int fa_perm(int r) {
 
 constexpr int FA_TK = 64;             // keys per tile
 constexpr int FA_TILE = FA_TK * 128;  // bytes of one K (or V^T) tile
-constexpr int FA_STAGE = 2 * FA_TILE;
 constexpr int FA_NS = 3;
 constexpr int kFaOOB = (int)0x80000000;
 
@@ -306,10 +305,26 @@ __device__ __forceinline__ float fa_sum_halves(float x) {
 // NWV waves per workgroup (4: 128 queries; 2: 64 queries for grids that
 // would otherwise leave SIMDs with a single wave).  Each wave issues 8 / NWV
 // of the 8-row DMA groups of every K and V^T tile.
-template <int NWV>
+// DG: head size in groups of 8 (8: the 64 of every SDXL layer).  The score
+// product runs over DK steps of 16 (a last half step reads zeros), P V over DV
+// blocks of 32 rows of V^T (rows past the head size hold whatever the LDS
+// held; they end in output rows that are never stored).  A head of 80 keeps
+// its dims 64-79 in a second K tile of 32-byte rows, so the first stays
+// 128 bytes wide.
+// Head sizes other than 64 scale the scores in fp32 after the MFMA (one more
+// multiply per score) instead of rounding scale * Q to fp16: the path they
+// replace held its scores in fp32.
+template <int NWV, int DG>
 __global__ void __launch_bounds__(NWV * 64) __attribute__((amdgpu_waves_per_eu(2)))
 flash_vt_pipe_kernel(FlashVtParams p) {
   constexpr int DI = 8 / NWV;  // DMA instructions per wave per operand tile
+  constexpr int DK = (DG + 1) / 2, DV = (DG + 3) / 4;
+  constexpr int IV = (DG + NWV - 1) / NWV;  // the same for the V^T tile (8 rows each)
+  constexpr bool K2 = DG > 8;
+  static_assert(DG <= 10, "at most 16 dims in the second K tile");
+  constexpr bool QS = DG == 8;  // scale folded into Q
+  constexpr int FA_VT = FA_TILE + (K2 ? 2048 : 0);  // byte offset of the V^T tile in a stage
+  constexpr int FA_STAGE = FA_VT + DV * 32 * 128;
   __shared__ __attribute__((aligned(1024))) unsigned char smem_g[FA_NS * FA_STAGE];
   unsigned char DLM_LDS* smem = (unsigned char DLM_LDS*)smem_g;
   // XCD-aware placement: the hardware deals workgroup i to XCD i % 8 and each
@@ -332,20 +347,29 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   const int g = lane >> 5;
   const int q0 = qb * (NWV * 32) + wave * 32;
 
-  f16x8 qf[4];  // this wave's 32 queries, loaded below
+  f16x8 qf[DK];  // this wave's 32 queries, loaded below
   const i32x4 rk = fa_rsrc(p.k, p.k_bytes);
   const i32x4 rv = fa_rsrc(p.vt, p.vt_bytes);
   // DMA instruction i of this wave: LDS row r of the tile, 16-byte chunk c of
   // it; the K row holds key fa_perm(r), the V^T row's chunk keys 8c .. 8c+7
   auto dma_row = [&](int i) { return (wave * DI + i) * 8 + (lane >> 3); };
   auto dma_chunk = [&](int r) { return (lane & 7) ^ ((r >> 1) & 7); };
-  int koff[DI], voff[DI];
+  auto dma_vrow = [&](int i) { return DG == 8 ? dma_row(i) : (i * NWV + wave) * 8 + (lane >> 3); };
+  int koff[DI], voff[IV], k2off = 0;
 #pragma unroll
   for (int i = 0; i < DI; ++i) {
     const int r = dma_row(i), c = dma_chunk(r);
     koff[i] = (int)((b * p.k_sb + h * p.k_sh + (long long)fa_perm(r) * p.k_ss + c * 8) * 2);
+    if (DG < 8 && c >= DG) koff[i] = kFaOOB;  // stays past the buffer in every tile
+  }
+#pragma unroll
+  for (int i = 0; i < IV; ++i) {
+    const int r = dma_vrow(i), c = dma_chunk(r);
     voff[i] = (int)((b * p.vt_sb + h * p.vt_sh + (long long)r * p.vt_ld + c * 8) * 2);
   }
+  const int k2row = (wave & 1) * 32 + (lane >> 1);  // waves 0 and 1: rows of the second K tile
+  if constexpr (K2)
+    k2off = (int)((b * p.k_sb + h * p.k_sh + (long long)fa_perm(k2row) * p.k_ss + 64 + (lane & 1) * 8) * 2);
   const int kstep = (int)(FA_TK * p.k_ss * 2);
   // keys past Sk exist only in a partial last tile; their rows and chunks are
   // recomputed there rather than held in registers for the whole loop
@@ -355,9 +379,13 @@ flash_vt_pipe_kernel(FlashVtParams p) {
     if (k0 + FA_TK <= p.Sk) {  // a full tile (all but a partial last one): no masking
 #pragma unroll
       for (int i = 0; i < DI; ++i) fa_dma16(rk, st + (wave * DI + i) * 1024, koff[i] + kt * kstep);
+      if constexpr (K2) {
+        if (wave < 2) fa_dma16(rk, st + FA_TILE + wave * 1024, k2off + kt * kstep);
+      }
 #pragma unroll
-      for (int i = 0; i < DI; ++i)
-        fa_dma16(rv, st + FA_TILE + (wave * DI + i) * 1024, voff[i] + kt * (FA_TK * 2));
+      for (int i = 0; i < IV; ++i)
+        if (DG == 8 || i * NWV + wave < DG)
+          fa_dma16(rv, st + FA_VT + (DG == 8 ? wave * DI + i : i * NWV + wave) * 1024, voff[i] + kt * (FA_TK * 2));
       return;
     }
 #pragma unroll
@@ -365,10 +393,16 @@ flash_vt_pipe_kernel(FlashVtParams p) {
       const bool in = k0 + fa_perm(dma_row(i)) < p.Sk;
       fa_dma16(rk, st + (wave * DI + i) * 1024, in ? koff[i] + kt * kstep : kFaOOB);
     }
+    if constexpr (K2) {
+      if (wave < 2)
+        fa_dma16(rk, st + FA_TILE + wave * 1024, k0 + fa_perm(k2row) < p.Sk ? k2off + kt * kstep : kFaOOB);
+    }
 #pragma unroll
-    for (int i = 0; i < DI; ++i) {
-      const bool in = k0 + dma_chunk(dma_row(i)) * 8 < p.Sk;
-      fa_dma16(rv, st + FA_TILE + (wave * DI + i) * 1024, in ? voff[i] + kt * (FA_TK * 2) : kFaOOB);
+    for (int i = 0; i < IV; ++i) {
+      const bool in = k0 + dma_chunk(dma_vrow(i)) * 8 < p.Sk;
+      if (DG == 8 || i * NWV + wave < DG)
+        fa_dma16(rv, st + FA_VT + (DG == 8 ? wave * DI + i : i * NWV + wave) * 1024,
+                 in ? voff[i] + kt * (FA_TK * 2) : kFaOOB);
     }
   };
   auto frag = [&](const unsigned char DLM_LDS* st, int row, int chunk) -> f16x8 {
@@ -383,15 +417,20 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   // The two key blocks' chains alternate, so consecutive MFMAs are
   // independent and VALU work can issue between dependent ones.
   auto scores = [&](const unsigned char DLM_LDS* st, f32x16 (&sv)[2], const f32x16& init) {
-    f16x8 kf[2][4];
+    f16x8 kf[2][DK];
 #pragma unroll
-    for (int ds = 0; ds < 4; ++ds)
+    for (int ds = 0; ds < DK; ++ds)
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) kf[kb][ds] = frag(st, kb * 32 + (lane & 31), 2 * ds + g);
+      for (int kb = 0; kb < 2; ++kb) {
+        if (ds < 4)
+          kf[kb][ds] = frag(st, kb * 32 + (lane & 31), 2 * ds + g);
+        else
+          kf[kb][ds] = *reinterpret_cast<const f16x8 DLM_LDS*>(st + FA_TILE + (kb * 32 + (lane & 31)) * 32 + g * 16);
+      }
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) sv[kb] = mfma32x32x16(kf[kb][0], qf[0], init);
 #pragma unroll
-    for (int ds = 1; ds < 4; ++ds)
+    for (int ds = 1; ds < DK; ++ds)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) sv[kb] = mfma32x32x16(kf[kb][ds], qf[ds], sv[kb]);
   };
@@ -412,18 +451,20 @@ flash_vt_pipe_kernel(FlashVtParams p) {
     const int qi = q0 + (lane & 31);
     const bool qin = qi < p.Sq;
     const f16* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)(qin ? qi : p.Sq - 1) * p.q_ss + g * 8;
-    f16x8 v[4];
+    f16x8 v[DK];
 #pragma unroll
-    for (int ds = 0; ds < 4; ++ds) v[ds] = *reinterpret_cast<const f16x8*>(qp + ds * 16);
-    const float cq = qin ? p.c : 0.0f;
+    for (int ds = 0; ds < DK; ++ds)  // a half step past the head size re-reads the first dims, times 0
+      v[ds] = *reinterpret_cast<const f16x8*>(2 * ds + 1 < DG || g == 0 ? qp + ds * 16 : qp - g * 8);
+    const float cq = qin ? (QS ? p.c : (p.c < 0.0f ? -1.0f : 1.0f)) : 0.0f;
 #pragma unroll
-    for (int ds = 0; ds < 4; ++ds) {
+    for (int ds = 0; ds < DK; ++ds) {
+      const float cd = 2 * ds + 1 < DG || g == 0 ? cq : 0.0f;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) v[ds][t] = (f16)((float)v[ds][t] * cq);
+      for (int t = 0; t < 8; ++t) v[ds][t] = (f16)((float)v[ds][t] * cd);
       qf[ds] = v[ds];
     }
   }
-
+  const float cs = QS ? 1.0f : fabsf(p.c);  // log2 units per score
 
   // Running state, in log2 units: the scores of a tile arrive as s - m with m
   // the lane's current base (negm = -m broadcast is every score chain's
@@ -433,18 +474,18 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   // base it re-bases them too.
   float l_run = 0.0f;
   f32x16 negm;
-  f32x16 o[2];
+  f32x16 o[DV];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    o[0][e] = 0.0f;
-    o[1][e] = 0.0f;
-  }
+  for (int dt = 0; dt < DV; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
 
   // p = 2^s of the 16 scores of one key block into two P fragments
   auto exp_block = [&](const f32x16& sk, f16x8& p0, f16x8& p1) {
 #pragma unroll
     for (int e = 0; e < 16; e += 2) {
-      const f16x2 hr = f16x2{(f16)__builtin_amdgcn_exp2f(sk[e]), (f16)__builtin_amdgcn_exp2f(sk[e + 1])};
+      const f16x2 hr = QS ? f16x2{(f16)__builtin_amdgcn_exp2f(sk[e]), (f16)__builtin_amdgcn_exp2f(sk[e + 1])}
+                          : f16x2{(f16)__builtin_amdgcn_exp2f(sk[e] * cs), (f16)__builtin_amdgcn_exp2f(sk[e + 1] * cs)};
       f16x8& d8 = e < 8 ? p0 : p1;
       d8[e & 7] = hr[0];
       d8[(e & 7) + 1] = hr[1];
@@ -486,12 +527,13 @@ flash_vt_pipe_kernel(FlashVtParams p) {
         for (int e = 0; e < 16; ++e) mt = fmaxf(mt, sv[kb][e]);
       mt = fa_max_halves(mt);
       const float d = first ? mt : fmaxf(mt, 0.0f);
-      const float alpha = __builtin_amdgcn_exp2f(-d);
+      // (the first tile's state is zero; its d may be so low that 2^-d is inf)
+      const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(QS ? -d : -d * cs);
       l_run *= alpha;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        o[0][e] *= alpha;
-        o[1][e] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < DV; ++dt) o[dt][e] *= alpha;
         negm[e] -= d;
       }
 #pragma unroll
@@ -511,21 +553,21 @@ flash_vt_pipe_kernel(FlashVtParams p) {
     l_run += lsum;
   };
   // O^T += V^T P^T over four 16-key steps (step j: tile keys 16j + 8g + [0, 8))
-  auto pv = [&](const f16x8 (&vf)[8], const f16x8 (&pf)[4]) {
+  auto pv = [&](const f16x8 (&vf)[4 * DV], const f16x8 (&pf)[4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt) o[dt] = mfma32x32x16(vf[j * 2 + dt], pf[j], o[dt]);
+      for (int dt = 0; dt < DV; ++dt) o[dt] = mfma32x32x16(vf[j * DV + dt], pf[j], o[dt]);
   };
-  auto vread = [&](const unsigned char DLM_LDS* st, f16x8 (&vf)[8]) {
+  auto vread = [&](const unsigned char DLM_LDS* st, f16x8 (&vf)[4 * DV]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt) vf[j * 2 + dt] = frag(st + FA_TILE, dt * 32 + (lane & 31), 2 * j + g);
+      for (int dt = 0; dt < DV; ++dt) vf[j * DV + dt] = frag(st + FA_VT, dt * 32 + (lane & 31), 2 * j + g);
   };
 
   // prologue: tile 0 published, its scores issued
-  if (nkt > 1) {
+  if (DG == 8 && nkt > 1) {  // (other head sizes: the waves issue unequal numbers)
     FA_WAIT_VM(2 * DI);  // tile 1's requests may still be in flight
   } else {
     FA_WAIT_VM(0);
@@ -546,7 +588,7 @@ flash_vt_pipe_kernel(FlashVtParams p) {
     if (kt + 2 < nkt) issue(nn, kt + 2);
     const unsigned char DLM_LDS* st = smem + c * FA_STAGE;
     scores(smem + nxt * FA_STAGE, sn, negm);  // tile kt+1, in the shadow of the softmax below
-    f16x8 vf[8];
+    f16x8 vf[4 * DV];
     vread(st, vf);
     f16x8 pf[4];
     // the instruction mix of the block up to the growth branch, interleaved:
@@ -574,7 +616,7 @@ flash_vt_pipe_kernel(FlashVtParams p) {
         for (int e = 0; e < 16; ++e)
           if (kb * 32 + 16 * (e >> 3) + 4 * ((e >> 2) & 1) + (e & 3) >= lim) sc[kb][e] = -INFINITY;
     }
-    f16x8 vf[8];
+    f16x8 vf[4 * DV];
     vread(smem + cur * FA_STAGE, vf);
     f16x8 pf[4];
     softmax(sc, pf, nullptr, kt == 0);
@@ -621,21 +663,24 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   const float l_tot = fa_sum_halves(l_run);
   const float inv = 1.0f / l_tot;
   __syncthreads();  // every wave is done reading the K / V^T ring
-  unsigned char DLM_LDS* ob = smem + wave * 4096;  // this wave's 32 rows x 128 B, chunks swizzled
+  // this wave's 32 rows x DG chunks of 16 bytes (64 dims: chunks swizzled)
+  unsigned char DLM_LDS* ob = smem + wave * (32 * DG * 16);
+  auto sw = [&](int row) { return DG == 8 ? row & 7 : 0; };
 #pragma unroll
-  for (int dt = 0; dt < 2; ++dt)
+  for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
     for (int gq = 0; gq < 4; ++gq) {
+      const int chunk = dt * 4 + gq;
+      if (chunk >= DG) continue;
       f16x4 r;
 #pragma unroll
       for (int t = 0; t < 4; ++t) r[t] = (f16)(o[dt][4 * gq + t] * inv);
-      const int chunk = dt * 4 + gq;
-      *reinterpret_cast<f16x4 DLM_LDS*>(ob + ql * 128 + ((chunk ^ (ql & 7)) * 16) + g * 8) = r;
+      *reinterpret_cast<f16x4 DLM_LDS*>(ob + ql * (DG * 16) + ((chunk ^ sw(ql)) * 16) + g * 8) = r;
     }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = i * 4 + (lane >> 4), piece = lane & 15;
-    const f16x4 r = *reinterpret_cast<const f16x4 DLM_LDS*>(ob + row * 128 + (((piece >> 1) ^ (row & 7)) * 16) +
+  for (int i = 0; i < DG; ++i) {
+    const int idx = i * 64 + lane, row = idx / (2 * DG), piece = idx - row * (2 * DG);
+    const f16x4 r = *reinterpret_cast<const f16x4 DLM_LDS*>(ob + row * (DG * 16) + (((piece >> 1) ^ sw(row)) * 16) +
                                                              (piece & 1) * 8);
     const int qi = q0 + row;
     if (qi < p.Sq)
@@ -643,7 +688,26 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   }
 }
 
-int attention_vt(const dlm_attention_vt_args* a, hipStream_t s) {
+template <int DG>
+static int launch_flash(FlashVtParams& p, hipStream_t s) {
+  // Cross attention (every key in at most two tiles): always 128-query
+  // workgroups, whose one K/V staging serves twice the queries.
+  const long long bh = (long long)p.H * p.B;
+  static const std::string n2 = "flash_vt_pipe_kernel<2, " + std::to_string(DG) + ">";
+  static const std::string n4 = "flash_vt_pipe_kernel<4, " + std::to_string(DG) + ">";
+  if (p.Sk > 2 * FA_TK && (p.Sq + 127) / 128 * bh < 512) {
+    p.nqb = (p.Sq + 63) / 64;
+    DLM_LAUNCH(n2.c_str(), (flash_vt_pipe_kernel<2, DG>), dim3(p.nqb * p.H * p.B), dim3(128), 0, s, p);
+  } else {
+    p.nqb = (p.Sq + 127) / 128;
+    DLM_LAUNCH(n4.c_str(), (flash_vt_pipe_kernel<4, DG>), dim3(p.nqb * p.H * p.B), dim3(256), 0, s, p);
+  }
+  DLM_LAUNCH_CHECK();
+  return DLM_OK;
+}
+
+// Head size Dh is 40, 64 or 80 (the callers check).
+static int attention_vt(const dlm_attention_vt_args* a, int Dh, hipStream_t s) {
   FlashVtParams p;
   p.q = (const f16*)a->q;
   p.k = (const f16*)a->k;
@@ -663,22 +727,12 @@ int attention_vt(const dlm_attention_vt_args* a, hipStream_t s) {
   // two query blocks (2x4096^2 x10 heads: 144 us vs 170 us).  Grids of fewer
   // than two 128-query workgroups per CU (1024 tokens x 20 heads x 2) take
   // 64-query workgroups: twice the K/V staging, but waves spread evenly.
-  // Cross attention (every key in at most two tiles): always 128-query
-  // workgroups, whose one K/V staging serves twice the queries.
   p.H = a->H;
   p.B = a->B;
   // the 1-D grid counts query blocks x heads x batch in int (host and kernel)
   if ((long long)((a->Sq + 63) / 64) * a->H * a->B >= (1LL << 31))
     return fail(DLM_ERR_UNSUPPORTED, "attention: more than 2^31 query blocks x heads x batch");
-  if (a->Sk > 2 * FA_TK && (long long)((a->Sq + 127) / 128) * a->H * a->B < 512) {
-    p.nqb = (a->Sq + 63) / 64;
-    DLM_LAUNCH("flash_vt_pipe_kernel<2>", flash_vt_pipe_kernel<2>, dim3(p.nqb * p.H * p.B), dim3(128), 0, s, p);
-  } else {
-    p.nqb = (a->Sq + 127) / 128;
-    DLM_LAUNCH("flash_vt_pipe_kernel<4>", flash_vt_pipe_kernel<4>, dim3(p.nqb * p.H * p.B), dim3(256), 0, s, p);
-  }
-  DLM_LAUNCH_CHECK();
-  return DLM_OK;
+  return Dh == 64 ? launch_flash<8>(p, s) : Dh == 40 ? launch_flash<5>(p, s) : launch_flash<10>(p, s);
 }
 
 int attention_strided(const dlm_attention_args* a, hipStream_t s) {
@@ -883,22 +937,27 @@ static int attention_reference_layout(const f16* q, const f16* k, const f16* v, 
   const long long BH = (long long)B * H;
   const int K8 = (Sk + 7) & ~7;
   int st = DLM_OK;
-  if (Dh == 64 && dlm_aligned16(q) && dlm_aligned16(k) && ((uintptr_t)o & 7) == 0) {
-    f16* vt = (f16*)scratch_slot((size_t)BH * 64 * K8 * 2, 6, s, &st);
+  // Head sizes of the SD and SDXL UNets: the flash kernel (2 x 10 heads x 2259
+  // tokens x 80: 77 us against 969 us for a GEMM, softmax and GEMM per head).
+  // Any other size, and operands that are not aligned, take those per head.
+  const bool vt_fits = (unsigned long long)BH * Dh * K8 * 2 < (1ull << 31);
+  if ((Dh == 64 || ((Dh == 40 || Dh == 80) && vt_fits)) && dlm_aligned16(q) && dlm_aligned16(k) &&
+      ((uintptr_t)o & 7) == 0) {
+    f16* vt = (f16*)scratch_slot((size_t)BH * Dh * K8 * 2, 6, s, &st);
     if (!vt) return st;
-    if ((st = vt_pad(v, vt, BH, Sk, 64, K8, s)) != DLM_OK) return st;
+    if ((st = vt_pad(v, vt, BH, Sk, Dh, K8, s)) != DLM_OK) return st;
     dlm_attention_vt_args a{};
     a.q = q; a.k = k; a.vt = vt; a.o = o;
-    a.q_sh = (long long)Sq * 64; a.q_sb = a.q_sh * H; a.q_ss = 64;
-    a.k_sh = (long long)Sk * 64; a.k_sb = a.k_sh * H; a.k_ss = 64;
-    a.vt_sh = 64LL * K8; a.vt_sb = a.vt_sh * H; a.vt_ld = K8;
-    a.o_sh = (long long)Sq * 64; a.o_sb = a.o_sh * H; a.o_ss = 64;
+    a.q_sh = (long long)Sq * Dh; a.q_sb = a.q_sh * H; a.q_ss = Dh;
+    a.k_sh = (long long)Sk * Dh; a.k_sb = a.k_sh * H; a.k_ss = Dh;
+    a.vt_sh = (long long)Dh * K8; a.vt_sb = a.vt_sh * H; a.vt_ld = K8;
+    a.o_sh = (long long)Sq * Dh; a.o_sb = a.o_sh * H; a.o_ss = Dh;
     a.B = B; a.H = H; a.Sq = Sq; a.Sk = Sk; a.scale = scale;
-    a.k_bytes = (unsigned long long)BH * Sk * 64 * 2;
-    a.vt_bytes = (unsigned long long)BH * 64 * K8 * 2;
+    a.k_bytes = (unsigned long long)BH * Sk * Dh * 2;
+    a.vt_bytes = (unsigned long long)BH * Dh * K8 * 2;
     if (a.k_bytes >= (1ull << 31) || a.vt_bytes >= (1ull << 31))
       return fail(DLM_ERR_UNSUPPORTED, "attention: K or V larger than 2 GiB");
-    return attention_vt(&a, s);
+    return attention_vt(&a, Dh, s);
   }
   const int D8 = (Dh + 7) & ~7;
   const int K4 = (Sk + 3) & ~3;
@@ -985,7 +1044,7 @@ int dlm_attention_vt_fp16(const dlm_attention_vt_args* a, void* stream) {
   const long long vlast = ((a->B - 1) * a->vt_sb + (a->H - 1) * a->vt_sh + 63LL * a->vt_ld + sk8) * 2;
   DLM_REQUIRE(klast <= (long long)a->k_bytes && vlast <= (long long)a->vt_bytes,
               "K or V^T extends past its buffer size");
-  return attention_vt(a, (hipStream_t)stream);
+  return attention_vt(a, 64, (hipStream_t)stream);
 }
 
 int dlm_softmax_rows_f32_fp16(const float* S, long long lds, void* P, long long ldp, int rows,

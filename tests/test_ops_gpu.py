@@ -328,6 +328,24 @@ def test_attention_reference_api_any_head_dim(gpu, B, H, Sq, Sk, Dh):
     assert_close(out, ref, f"attention Dh={Dh}")
 
 
+@pytest.mark.parametrize("Dh", [40, 80])
+@pytest.mark.parametrize("B,H,Sq,Sk,mul", [(1, 1, 1, 1, 1.0), (2, 2, 31, 64, 1.0), (1, 3, 129, 65, 1.0),
+                                           (2, 10, 333, 511, 1.0), (1, 20, 600, 1029, 1.0), (1, 2, 96, 200, -1.0),
+                                           (1, 2, 70, 450, 24.0)])
+def test_attention_flash_head_dims(gpu, B, H, Sq, Sk, Dh, mul):
+    """Head sizes 40 and 80 on the flash kernel: partial query blocks and key tiles, both workgroup
+    widths, every ring position of the last tile, a negative scale, and scores that move the softmax
+    base (24 / sqrt(Dh))."""
+    announce(f"launch_attention flash B={B} H={H} Sq={Sq} Sk={Sk} Dh={Dh} x{mul}")
+    q, k, v = randn((B, H, Sq, Dh), 113), randn((B, H, Sk, Dh), 114), randn((B, H, Sk, Dh), 115)
+    scale = mul / math.sqrt(Dh)
+    out = torch.full((B, H, Sq, Dh), 7.0, dtype=torch.float16, device=gpu)
+    ops.launch_attention(to_gpu(q), to_gpu(k), to_gpu(v), out, B, H, Sq, Sk, Dh, scale)
+    ref = torch.cat([R.attention(q[b:b + 1], k[b:b + 1], v[b:b + 1], scale) for b in range(B)])
+    # P and O are rounded to fp16 (half a unit in 2^11 each, relative)
+    assert float((out.float().cpu() - ref).norm() / ref.norm()) <= 1e-3
+
+
 def test_attention_reference_api_unaligned(gpu):
     """Q / K / V / O that start 2 bytes into their allocation take the general path."""
     B, H, Sq, Sk, Dh = 1, 2, 70, 45, 64
