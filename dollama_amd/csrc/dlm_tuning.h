@@ -32,7 +32,8 @@ extern "C" {
  * 39 128x64 64x32 3; 40 128x128 32x64 2 and 41 256x160 32x160 3 with the
  * next slice's first fragments read early; 42 128x16 16x16 3 and 43 64x16
  * 16x16 3 (outputs of at most 16 columns); 44 192x160 48x80 3 (at most 192
- * rows, e.g. the text tokens' K/V projection).  Splits apply to the LDS-DMA core
+ * rows, e.g. the text tokens' K/V projection); 45 256x160 64x80 3 in
+ * ping-pong.  Splits apply to the LDS-DMA core
  * only. */
 int dlm_gemm_force_tile(int tile_id);
 /* Same override for GEMMs / convs of one shape (M, N = output columns,
@@ -41,9 +42,8 @@ int dlm_gemm_force_tile(int tile_id);
  * only launches made by the calling thread. */
 int dlm_gemm_override_shape(int M, int N, int K, int tile_id, int splits);
 int dlm_gemm_force_split(int splits);
-/* Tuning aid: select alternative tile heuristics (0 = default; bit 0 = no
- * 160-column / split-K rules; bit 1 = no fragment-prefetch forms, four
- * splits for 256x160 grids that fill the chip). */
+/* Tuning aid: select alternative tile heuristics (0 = default; bit 0 = plans
+ * without split-K). */
 int dlm_gemm_set_variant(int variant);
 
 /* Counter calibration: `blocks` workgroups of 4 waves, each wave `iters`

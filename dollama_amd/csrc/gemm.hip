@@ -43,6 +43,8 @@
 namespace dlm {
 
 constexpr int BK = 64;
+// Main-loop schedules of dma_gemm_kernel (described there)
+constexpr int kPlain = 0, kPrefetch = 1, kPingPong = 2;
 constexpr int LS = BK + 8;  // LDS row stride in halfs
 
 struct EpiArgs {
@@ -1118,11 +1120,25 @@ __device__ __forceinline__ void split_coords(int bid, int tiles_m, int tiles_n, 
   tn = rem / gsz;
 }
 
-// PF: the first k-step's fragments of slice kt+1 are read from LDS right
+// SCH kPrefetch: the first k-step's fragments of slice kt+1 are read from LDS right
 // after the barrier that publishes it, while the second k-step of slice kt
 // (already in registers) runs on the MFMA pipe; the whole ring is filled
 // before the loop and slot kt is refilled (with slice kt+NS) as soon as that
 // barrier proves every wave has read it.
+// SCH kPingPong (two waves per SIMD, the second half of the waves one barrier
+// behind the first): between two barriers one half reads its fragments and
+// issues DMA while the other half, on the same SIMDs, issues nothing but MFMAs,
+// so the LDS port and the matrix pipe work at the same time instead of in
+// turn.  Reads of slice kt end (lgkmcnt(0)) before the barrier that closes
+// their phase, and the last of them (the late half's second k-step) before the
+// first phase that refills the slot, one slice later.  A wave waits for its own
+// part of slice kt+1 in the second read phase of slice kt, a barrier before
+// either half reads it.  256x160 tile, 64x80 waves: 1690 cycles a slice, of
+// which the MFMAs are 1280 (1290 with the DMA or the reads taken out), at the
+// 1.6 GHz that the power limit leaves; the plain loop needs 10% more.
+// 2048x10240x1280 GEGLU 71 -> 65 us, 4096x2560x5120 112 -> 100 us.  Smaller
+// tiles, whose read phases are longer than their MFMA phases, measured slower
+// with it (128x128: 29 -> 34 us at 2048x3840x1280).
 // SPS > 1: a ring stage holds SPS consecutive K slices published by one
 // barrier (fewer barriers and exposed first reads per slice); slices past the
 // range end are loaded clamped and skipped by the MFMAs.
@@ -1130,7 +1146,7 @@ __device__ __forceinline__ void split_coords(int bid, int tiles_m, int tiles_n, 
 // rows from the A fragments it multiplies (two v_dot2 per 4 halves, fp32
 // accumulation of exact fp16 products); the four lanes that hold one row's
 // K chunks combine their sums after the loop.  No split-K.
-template <int BM, int BN, int WM, int WN, int NS, bool PF, int SPS, bool LNS, class Desc>
+template <int BM, int BN, int WM, int WN, int NS, int SCH, int SPS, bool LNS, class Desc>
 __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64)
 dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, SplitArgs sp) {
   constexpr int WAVES_N = BN / WN;
@@ -1144,7 +1160,7 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
   constexpr int IA = (GA + NW - 1) / NW, IB = (GB + NW - 1) / NW;  // DMA instructions per wave
   static_assert(BM % 8 == 0 && BN % 8 == 0 && WM % 16 == 0 && WN % 16 == 0, "tile shape");
   static_assert(NS >= 2, "at least two slices");
-  static_assert(SPS == 1 || !PF, "multi-slice stages use the plain loop");
+  static_assert(SPS == 1 || SCH == kPlain, "multi-slice stages use the plain loop");
   __shared__ __attribute__((aligned(1024))) unsigned char smem_generic[NS * STAGE];
   unsigned char DLM_LDS* smem = (unsigned char DLM_LDS*)smem_generic;
 
@@ -1226,7 +1242,7 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
   f16x4 ebv[TN], erv[TM][TN];
   bool early = false;
 
-  constexpr int PRE = SPS > 1 ? 0 : (PF ? NS : NS - 1);  // slices in flight before the loop
+  constexpr int PRE = SPS > 1 ? 0 : (SCH == kPrefetch ? NS : NS - 1);  // slices in flight before the loop
 #pragma unroll
   for (int s = 0; s < PRE; ++s) issue_all(s, min(kb + s, ke - 1));
 
@@ -1338,7 +1354,60 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
       slot = slot + 1 == NS ? 0 : slot + 1;
       nslot = nslot + 1 == NS ? 0 : nslot + 1;
     }
-  } else if constexpr (PF) {
+  } else if constexpr (SCH == kPingPong) {
+    const bool late = wave >= NW / 2;
+    // byte offset of this lane's first A / B fragment within a stage, k-step 0
+    const int l15 = lane & 15, fc = ((lane >> 4) ^ (l15 >> 1)) * 16;
+    const int fa0 = (wm * WM + l15) * 128 + fc, fb0 = SA + (wn * WN + l15) * 128 + fc;
+    DLM_WAIT_SLICES(NS - 2);  // slice kb
+    __builtin_amdgcn_s_barrier();
+    if (late) __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    int slot = 0, nslot = NS - 1;
+    for (int kt = kb; kt < ke; ++kt) {
+      const unsigned char DLM_LDS* st = smem + slot * STAGE;
+      unsigned char DLM_LDS* nst = smem + nslot * STAGE;
+      const int nkt = min(kt + NS - 1, ke - 1);
+      al.prepare(nkt);
+      bl.prepare(nkt);
+      f16x8 fa[TM], fb[TN];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const unsigned char DLM_LDS* pa = st + (fa0 ^ (ks * 64));
+        const unsigned char DLM_LDS* pb = st + (fb0 ^ (ks * 64));
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const f16x8 DLM_LDS*>(pa + i * 2048);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const f16x8 DLM_LDS*>(pb + j * 2048);
+#pragma unroll
+        for (int i = 0; i < IA; ++i)
+          if (i % KS == ks) dma_a(nst, i, nkt);
+#pragma unroll
+        for (int i = 0; i < IB; ++i)
+          if ((IA + i) % KS == ks) dma_b(nst, i, nkt);
+        if (ks == KS - 1) DLM_WAIT_SLICES(NS - 2);  // slice kt+1
+        __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x32(fb[j], fa[i], acc[i][j]);
+        ln_acc(fa);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      slot = slot + 1 == NS ? 0 : slot + 1;
+      nslot = nslot + 1 == NS ? 0 : nslot + 1;
+    }
+    if (!late) __builtin_amdgcn_s_barrier();
+  } else if constexpr (SCH == kPrefetch) {
     static_assert(KS == 2, "prefetch form assumes two k-steps per slice");
     f16x8 f0a[TM], f0b[TN], f1a[TM], f1b[TN];
     auto rd = [&](const unsigned char DLM_LDS* st, int ks, f16x8 (&fa)[TM], f16x8 (&fb)[TN]) {
@@ -1436,21 +1505,23 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
   if (!LNS && sp.S > 1) {
     // ---- split-K reduction (last arriver) ----
     const int tile = tmi * tiles_n + tni;
-    constexpr int PER = BM * BN;  // floats per partial
-    float* mine = sp.ws + ((size_t)tile * sp.S + sidx) * PER;
-    const int base = (wave * TM * TN) * 256 + lane * 4;  // float index of block (0,0)
+    // Partials move in 16-byte accesses at agent scope (sc1: written through
+    // to, and read from, the point all XCDs share).
+    constexpr int kAgent = 16;      // cache-policy bit sc1
+    constexpr int PER = BM * BN * 4;  // bytes per partial
+    const int off = (wave * TM * TN * 64 + lane) * 16;  // byte offset of block (0,0)
+    auto part = [&](int sx) {
+      return make_rsrc(reinterpret_cast<const char*>(sp.ws) + ((size_t)tile * sp.S + sx) * PER, PER);
+    };
+    {
+      const rsrc_t mine = part(sidx);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        unsigned long long* p = reinterpret_cast<unsigned long long*>(mine + base + (i * TN + j) * 256);
-        const unsigned long long lo = ((unsigned long long)__float_as_uint(acc[i][j][1]) << 32) |
-                                      __float_as_uint(acc[i][j][0]);
-        const unsigned long long hi = ((unsigned long long)__float_as_uint(acc[i][j][3]) << 32) |
-                                      __float_as_uint(acc[i][j][2]);
-        __hip_atomic_store(p, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(p + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+        for (int j = 0; j < TN; ++j)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), mine, off,
+                                                 (i * TN + j) * 1024, kAgent);
+    }
     DLM_WAIT_VM(0);  // this wave's partial is complete at agent scope
     __syncthreads();  // every wave's partial complete, every fragment read done
     int* flag = reinterpret_cast<int*>(smem_generic);  // the operand ring is free now
@@ -1472,18 +1543,13 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
 #pragma unroll
           for (int j = 0; j < TN; ++j) tot[i][j] += acc[i][j];
       } else {
-        const float* other = sp.ws + ((size_t)tile * sp.S + s) * PER;
+        const rsrc_t other = part(s);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const unsigned long long* p =
-                reinterpret_cast<const unsigned long long*>(other + base + (i * TN + j) * 256);
-            const unsigned long long lo = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long hi = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            tot[i][j] += f32x4{__uint_as_float((unsigned)lo), __uint_as_float((unsigned)(lo >> 32)),
-                               __uint_as_float((unsigned)hi), __uint_as_float((unsigned)(hi >> 32))};
-          }
+          for (int j = 0; j < TN; ++j)
+            tot[i][j] += __builtin_bit_cast(
+                f32x4, __builtin_amdgcn_raw_buffer_load_b128(other, off, (i * TN + j) * 1024, kAgent));
       }
     }
     if (tid == 0) __hip_atomic_store(sp.cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1657,13 +1723,13 @@ struct NoSplitScope {
   ~NoSplitScope() { t_no_split = prev; }
 };
 
-// "dma_gemm_kernel<BM, BN, WM, WN, NS, PF, SPS, LNS, RowDesc|ConvDesc>", as
+// "dma_gemm_kernel<BM, BN, WM, WN, NS, SCH, SPS, LNS, RowDesc|ConvDesc>", as
 // the profiler prints the instantiation
-template <int BM, int BN, int WM, int WN, int NS, bool PF, int SPS, bool LNS, class Desc>
+template <int BM, int BN, int WM, int WN, int NS, int SCH, int SPS, bool LNS, class Desc>
 static const char* dma_kernel_name() {
   static const std::string n = "dma_gemm_kernel<" + std::to_string(BM) + ", " + std::to_string(BN) +
                                ", " + std::to_string(WM) + ", " + std::to_string(WN) + ", " +
-                               std::to_string(NS) + ", " + (PF ? "true" : "false") + ", " +
+                               std::to_string(NS) + ", " + std::to_string(SCH) + ", " +
                                std::to_string(SPS) + ", " + (LNS ? "true" : "false") + ", " +
                                (std::is_same<Desc, RowDesc>::value ? "RowDesc" : "ConvDesc") + ">";
   return n.c_str();
@@ -1672,9 +1738,9 @@ static const char* dma_kernel_name() {
 // Tile configurations with a LayerNorm-folding instantiation: the ones the
 // LayerNorm-consuming linears of the UNet take (2048- and 8192-row QKV, cross
 // Q and GEGLU shapes), plus their non-prefetch variants.
-template <int BM, int BN, int WM, int WN, int NS, bool PF, int SPS>
+template <int BM, int BN, int WM, int WN, int NS, int SCH, int SPS>
 constexpr bool ln_tile() {
-  return (BM == 128 && BN == 80 && WM == 16 && WN == 80 && NS == 3 && !PF && SPS == 2) ||
+  return (BM == 128 && BN == 80 && WM == 16 && WN == 80 && NS == 3 && SCH == kPlain && SPS == 2) ||
          (BM == 128 && BN == 128 && WM == 64 && WN == 32 && NS == 2 && SPS == 1) ||
          (BM == 128 && BN == 128 && WM == 32 && WN == 64 && NS == 2 && SPS == 1) ||
          (BM == 256 && BN == 160 && WM == 64 && WN == 80 && NS == 3 && SPS == 1) ||
@@ -1695,7 +1761,7 @@ static const char* mfma_kernel_name() {
 // point runs the statistics pass instead.
 static thread_local bool t_gn_written = false;
 
-template <int BM, int BN, int WM, int WN, int NS, bool PF = false, int SPS = 1, class Desc>
+template <int BM, int BN, int WM, int WN, int NS, int SCH = kPlain, int SPS = 1, class Desc>
 static int launch_dma(const Desc& ad, const RowDesc& bd, const EpiArgs& ep_in, int M, int N,
                       hipStream_t s, int S = 1) {
   static_assert(NS * SPS * (BM + BN) * BK * 2 <= 160 * 1024, "LDS ring larger than 160 KiB");
@@ -1725,11 +1791,11 @@ static int launch_dma(const Desc& ad, const RowDesc& bd, const EpiArgs& ep_in, i
   const int dims_flags = (ep.res ? 1 : 0) | (ep.act << 4) | (std::is_same<Desc, ConvDesc>::value ? 256 : 0) |
                          (ep.ln_c1 ? 512 : 0);
   if (ep.ln_c1) {
-    if constexpr (std::is_same<Desc, RowDesc>::value && ln_tile<BM, BN, WM, WN, NS, PF, SPS>()) {
+    if constexpr (std::is_same<Desc, RowDesc>::value && ln_tile<BM, BN, WM, WN, NS, SCH, SPS>()) {
       sp = SplitArgs{1, nk, nullptr, nullptr};
-      note_kernel(dma_kernel_name<BM, BN, WM, WN, NS, PF, SPS, true, Desc>());
+      note_kernel(dma_kernel_name<BM, BN, WM, WN, NS, SCH, SPS, true, Desc>());
       note_dims(M, N, bd.K, dims_flags);
-      launch((dma_gemm_kernel<BM, BN, WM, WN, NS, PF, SPS, true, Desc>), dim3(tiles), dim3(NT),
+      launch((dma_gemm_kernel<BM, BN, WM, WN, NS, SCH, SPS, true, Desc>), dim3(tiles), dim3(NT),
                          0, s, ad, bd, ep, tiles_m, tiles_n, sp);
       DLM_LAUNCH_CHECK();
       return DLM_OK;
@@ -1738,9 +1804,9 @@ static int launch_dma(const Desc& ad, const RowDesc& bd, const EpiArgs& ep_in, i
     }
   }
   const int grid = sp.S > 1 ? 8 * ((tiles + 7) / 8) * sp.S : tiles;
-  note_kernel(dma_kernel_name<BM, BN, WM, WN, NS, PF, SPS, false, Desc>());
+  note_kernel(dma_kernel_name<BM, BN, WM, WN, NS, SCH, SPS, false, Desc>());
   note_dims(M, N, bd.K, dims_flags);
-  launch((dma_gemm_kernel<BM, BN, WM, WN, NS, PF, SPS, false, Desc>), dim3(grid), dim3(NT), 0,
+  launch((dma_gemm_kernel<BM, BN, WM, WN, NS, SCH, SPS, false, Desc>), dim3(grid), dim3(NT), 0,
                      s, ad, bd, ep, tiles_m, tiles_n, sp);
   DLM_LAUNCH_CHECK();
   return DLM_OK;
@@ -1833,12 +1899,13 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
       if (!dma) return fail(DLM_ERR_UNSUPPORTED, "LayerNorm-folding GEMM needs aligned operands");
       switch (g_forced_tile) {  // tuning aid: the tiles with a folding kernel
         case 24: return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
-        case 28: return launch_dma<256, 160, 64, 80, 3, true>(ad, bd, ep, M, N, s);
-        case 29: return launch_dma<128, 128, 64, 32, 2, true>(ad, bd, ep, M, N, s);
-        case 31: return launch_dma<128, 160, 32, 80, 3, true>(ad, bd, ep, M, N, s);
-        case 35: return launch_dma<128, 80, 16, 80, 3, false, 2>(ad, bd, ep, M, N, s);
-        case 40: return launch_dma<128, 128, 32, 64, 2, true>(ad, bd, ep, M, N, s);
-        case 41: return launch_dma<256, 160, 32, 160, 3, true>(ad, bd, ep, M, N, s);
+        case 28: return launch_dma<256, 160, 64, 80, 3, kPrefetch>(ad, bd, ep, M, N, s);
+        case 29: return launch_dma<128, 128, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s);
+        case 31: return launch_dma<128, 160, 32, 80, 3, kPrefetch>(ad, bd, ep, M, N, s);
+        case 35: return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
+        case 40: return launch_dma<128, 128, 32, 64, 2, kPrefetch>(ad, bd, ep, M, N, s);
+        case 41: return launch_dma<256, 160, 32, 160, 3, kPrefetch>(ad, bd, ep, M, N, s);
+        case 45: return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s);
         case 0: break;
         default: return fail(DLM_ERR_UNSUPPORTED, "forced tile has no LayerNorm-folding kernel");
       }
@@ -1853,12 +1920,12 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
       const long long t160 = ceil_div(M, 128) * (N / 160);
       const int nk = (int)ceil_div(bd.K, BK);
       if (ep.act == DLM_ACT_GEGLU && N % 160 == 0 && t256 >= kCUs)
-        return launch_dma<256, 160, 32, 160, 3, true>(ad, bd, ep, M, N, s);
+        return launch_dma<256, 160, 32, 160, 3, kPrefetch>(ad, bd, ep, M, N, s);
       if (!ep.vt && ep.act != DLM_ACT_GEGLU && N % 80 == 0 && t80 >= kCUs * 3 / 4 && t80 <= kCUs)
-        return launch_dma<128, 80, 16, 80, 3, false, 2>(ad, bd, ep, M, N, s);
+        return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
       if (!ep.vt && ep.act != DLM_ACT_GEGLU && N % 160 == 0 && N <= 1280 && t160 >= kCUs && nk <= 100)
         return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
-      return launch_dma<128, 128, 32, 64, 2, true>(ad, bd, ep, M, N, s);
+      return launch_dma<128, 128, 32, 64, 2, kPrefetch>(ad, bd, ep, M, N, s);
     }
   }
   if (dma) {
@@ -1882,24 +1949,25 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
       case 24: return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
       case 25: return launch_dma<64, 160, 32, 80, 2>(ad, bd, ep, M, N, s);
       case 26: return launch_dma<128, 80, 16, 80, 5>(ad, bd, ep, M, N, s);
-      case 27: return launch_dma<128, 80, 16, 80, 5, true>(ad, bd, ep, M, N, s);
-      case 28: return launch_dma<256, 160, 64, 80, 3, true>(ad, bd, ep, M, N, s);
-      case 29: return launch_dma<128, 128, 64, 32, 2, true>(ad, bd, ep, M, N, s);
-      case 30: return launch_dma<128, 160, 32, 80, 4, true>(ad, bd, ep, M, N, s);
-      case 31: return launch_dma<128, 160, 32, 80, 3, true>(ad, bd, ep, M, N, s);
-      case 32: return launch_dma<256, 128, 64, 64, 3, true>(ad, bd, ep, M, N, s);
-      case 33: return launch_dma<128, 128, 64, 32, 4, true>(ad, bd, ep, M, N, s);
-      case 34: return launch_dma<128, 64, 64, 32, 2, true>(ad, bd, ep, M, N, s);
-      case 35: return launch_dma<128, 80, 16, 80, 3, false, 2>(ad, bd, ep, M, N, s);
-      case 36: return launch_dma<128, 80, 16, 80, 2, false, 2>(ad, bd, ep, M, N, s);
-      case 37: return launch_dma<128, 160, 32, 80, 2, false, 2>(ad, bd, ep, M, N, s);
-      case 38: return launch_dma<128, 128, 64, 32, 2, false, 2>(ad, bd, ep, M, N, s);
-      case 39: return launch_dma<128, 64, 64, 32, 3, false, 2>(ad, bd, ep, M, N, s);
-      case 40: return launch_dma<128, 128, 32, 64, 2, true>(ad, bd, ep, M, N, s);
-      case 41: return launch_dma<256, 160, 32, 160, 3, true>(ad, bd, ep, M, N, s);
+      case 27: return launch_dma<128, 80, 16, 80, 5, kPrefetch>(ad, bd, ep, M, N, s);
+      case 28: return launch_dma<256, 160, 64, 80, 3, kPrefetch>(ad, bd, ep, M, N, s);
+      case 29: return launch_dma<128, 128, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s);
+      case 30: return launch_dma<128, 160, 32, 80, 4, kPrefetch>(ad, bd, ep, M, N, s);
+      case 31: return launch_dma<128, 160, 32, 80, 3, kPrefetch>(ad, bd, ep, M, N, s);
+      case 32: return launch_dma<256, 128, 64, 64, 3, kPrefetch>(ad, bd, ep, M, N, s);
+      case 33: return launch_dma<128, 128, 64, 32, 4, kPrefetch>(ad, bd, ep, M, N, s);
+      case 34: return launch_dma<128, 64, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s);
+      case 35: return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
+      case 36: return launch_dma<128, 80, 16, 80, 2, kPlain, 2>(ad, bd, ep, M, N, s);
+      case 37: return launch_dma<128, 160, 32, 80, 2, kPlain, 2>(ad, bd, ep, M, N, s);
+      case 38: return launch_dma<128, 128, 64, 32, 2, kPlain, 2>(ad, bd, ep, M, N, s);
+      case 39: return launch_dma<128, 64, 64, 32, 3, kPlain, 2>(ad, bd, ep, M, N, s);
+      case 40: return launch_dma<128, 128, 32, 64, 2, kPrefetch>(ad, bd, ep, M, N, s);
+      case 41: return launch_dma<256, 160, 32, 160, 3, kPrefetch>(ad, bd, ep, M, N, s);
       case 42: return launch_dma<128, 16, 16, 16, 3>(ad, bd, ep, M, N, s);
       case 43: return launch_dma<64, 16, 16, 16, 3>(ad, bd, ep, M, N, s);
       case 44: return launch_dma<192, 160, 48, 80, 3>(ad, bd, ep, M, N, s);
+      case 45: return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s);
       default: break;
     }
     if (g_forced_tile == 0) {
@@ -1915,14 +1983,11 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
       // sit in lanes 16 apart, so any 16-column-multiple wave works).
       const long long t128 = ceil_div(M, 128) * ceil_div(N, 128);
       const bool pf = !(g_variant & 2);
-      // GEGLU FF1 at 2048x10240x1280: 256x160 tiles, three-slice ring, with
-      // fragment prefetch, measured in the whole UNet step in one process
-      // (25.3 ms against 26.0 with 128x128 and 26.7 with 256x128 for both FF1
-      // shapes).  Grids of four or more 256x160 tiles per CU (8192x5120x640)
-      // take the 128x128 prefetch tiles below: 0.11 ms less per step.
-      if (ep.act == DLM_ACT_GEGLU && N % 160 == 0 && ceil_div(M, 256) * (N / 160) >= kCUs &&
-          ceil_div(M, 256) * (N / 160) < 4 * kCUs)
-        return pf ? launch_dma<256, 160, 64, 80, 3, true>(ad, bd, ep, M, N, s)
+      // GEGLU with at least one 256x160 tile per CU: those, in ping-pong
+      // (2048x10240x1280 71 -> 65 us, 8192x5120x640 89 -> 79 us against
+      // the 128x128 prefetch tiles it took before).
+      if (ep.act == DLM_ACT_GEGLU && N % 160 == 0 && ceil_div(M, 256) * (N / 160) >= kCUs)
+        return pf ? launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s)
                   : launch_dma<256, 160, 64, 80, 3>(ad, bd, ep, M, N, s);
       // Output widths that are multiples of 160 (SDXL's 320 / 640 / 1280
       // channels): 160-column tiles give whole waves of tiles on 256 CUs
@@ -1944,16 +2009,16 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
       if ((std::is_same<Desc, RowDesc>::value || nk <= 100) && !ep.vt && N % 80 == 0 &&
           ceil_div(M, 128) * (N / 80) >= kCUs * 3 / 4 &&
           ceil_div(M, 128) * (N / 80) <= kCUs && !(g_variant & 1))
-        return launch_dma<128, 80, 16, 80, 3, false, 2>(ad, bd, ep, M, N, s);
+        return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
       if (!ep.vt && N % 160 == 0 && N <= 1280 && !(g_variant & 1)) {
         const long long t256 = ceil_div(M, 256) * (N / 160), t160 = ceil_div(M, 128) * (N / 160);
         if (t256 >= kCUs)
-          return launch_dma<256, 160, 64, 80, 3>(ad, bd, ep, M, N, s, !pf && nk >= 80 ? 4 : 1);
+          return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, !pf && nk >= 80 ? 4 : 1);
         if (t160 >= kCUs) {
           if (nk <= 100) return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
-          return launch_dma<256, 160, 64, 80, 3>(ad, bd, ep, M, N, s, 2);
+          return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, 2);
         } else if (nk >= 300 && t256 * 4 >= kCUs) {
-          return launch_dma<256, 160, 64, 80, 3>(ad, bd, ep, M, N, s, 4);
+          return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, 4);
         } else if (nk >= 44 && t160 * 4 >= kCUs) {
           return launch_dma<128, 160, 32, 80, 3>(ad, bd, ep, M, N, s, t160 * 2 >= kCUs ? 2 : 4);
         }
@@ -1972,13 +2037,16 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
                      ? launch_dma<128, 64, 64, 32, 2>(ad, bd, ep, M, N, s)
                      : launch_dma<128, 64, 64, 32, 4>(ad, bd, ep, M, N, s);
         // convolutions with one to four 128x128 tiles per CU: 256x128 tiles
-        // (fewer operand bytes per MFMA; the im2col loader is the costlier one)
+        // (fewer operand bytes per MFMA).  Larger grids keep 128x128, two
+        // workgroups to a CU, whose epilogues pass under each other's main
+        // loops (the VAE's 3x3 convs: 256x128 tiles 17.0 -> 17.4 ms a decode,
+        // although 4% faster on their own without the fp32 epilogue).
         if (std::is_same<Desc, ConvDesc>::value && t128 >= kCUs && t128 < 4 * kCUs)
           return launch_dma<256, 128, 64, 64, 3>(ad, bd, ep, M, N, s);
         // one workgroup's ring of two slices: the prefetch form (2048x3840x1280
         // QKV ~2 us faster per launch, 8192x1920x640 the same)
         if (t128 >= kCUs)
-          return pf ? launch_dma<128, 128, 64, 32, 2, true>(ad, bd, ep, M, N, s)
+          return pf ? launch_dma<128, 128, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s)
                     : launch_dma<128, 128, 64, 32, 2>(ad, bd, ep, M, N, s);
         return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s);
       }
@@ -2834,7 +2902,7 @@ extern "C" int dlm_gemm_override_shape(int M, int N, int K, int tile_id, int spl
 }
 
 extern "C" int dlm_gemm_force_tile(int tile_id) {
-  DLM_REQUIRE(tile_id >= 0 && tile_id <= 44, "tile_id must be in [0, 44]");
+  DLM_REQUIRE(tile_id >= 0 && tile_id <= 45, "tile_id must be in [0, 45]");
   dlm::g_forced_tile = tile_id;
   return DLM_OK;
 }
