@@ -1093,23 +1093,18 @@ struct SplitArgs {
   int* cnt;   // per-tile arrival counters, zero between launches
 };
 
-// blockIdx -> (tile, split) for S > 1: every split of a tile on one XCD
-// (workgroup b runs on XCD b % 8), XCDs own contiguous logical tile ranges,
-// logical tiles walk groups of 8 M-tiles as in tile_coords.  tm < 0 marks a
-// padding workgroup.
+// blockIdx -> (tile, split) for S > 1: the tiles' splits in one sequence, of
+// which each XCD (workgroup b runs on XCD b % 8) takes an equal contiguous
+// run, so no XCD gets more workgroups than it has CUs while others idle;
+// logical tiles walk groups of 8 M-tiles as in tile_coords.
 __device__ __forceinline__ void split_coords(int bid, int tiles_m, int tiles_n, int S, int& tm,
                                              int& tn, int& sidx) {
-  const int total = tiles_m * tiles_n;
-  const int q = (total + 7) >> 3;
-  const int x = bid & 7, slot = bid >> 3;
-  const int local = slot / S;
-  sidx = slot - local * S;
-  const int logical = x * q + local;
-  if (local >= q || logical >= total) {
-    tm = -1;
-    tn = 0;
-    return;
-  }
+  const int total = tiles_m * tiles_n * S;
+  const int q = total >> 3, r = total & 7;
+  const int x = bid & 7;
+  const int seq = x * q + (x < r ? x : r) + (bid >> 3);
+  const int logical = seq / S;
+  sidx = seq - logical * S;
   constexpr int GM = 8;
   const int per_group = GM * tiles_n;
   const int g = logical / per_group;
@@ -1171,7 +1166,6 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
   int tmi, tni, sidx = 0;
   if (sp.S > 1) {
     split_coords(blockIdx.x, tiles_m, tiles_n, sp.S, tmi, tni, sidx);
-    if (tmi < 0) return;
   } else {
     tile_coords(blockIdx.x, tiles_m, tiles_n, tmi, tni);
   }
@@ -1741,7 +1735,8 @@ static const char* dma_kernel_name() {
 template <int BM, int BN, int WM, int WN, int NS, int SCH, int SPS>
 constexpr bool ln_tile() {
   return (BM == 128 && BN == 80 && WM == 16 && WN == 80 && NS == 3 && SCH == kPlain && SPS == 2) ||
-         (BM == 128 && BN == 128 && WM == 64 && WN == 32 && NS == 2 && SPS == 1) ||
+         (BM == 128 && BN == 128 && WM == 64 && WN == 32 && SPS == 1) ||
+         (BM == 128 && BN == 64 && WM == 64 && WN == 32 && NS == 4 && SPS == 1) ||
          (BM == 128 && BN == 128 && WM == 32 && WN == 64 && NS == 2 && SPS == 1) ||
          (BM == 256 && BN == 160 && WM == 64 && WN == 80 && NS == 3 && SPS == 1) ||
          (BM == 256 && BN == 160 && WM == 32 && WN == 160 && NS == 3 && SPS == 1) ||
@@ -1803,7 +1798,7 @@ static int launch_dma(const Desc& ad, const RowDesc& bd, const EpiArgs& ep_in, i
       return fail(DLM_ERR_UNSUPPORTED, "LayerNorm-folding GEMM: tile without a folding kernel");
     }
   }
-  const int grid = sp.S > 1 ? 8 * ((tiles + 7) / 8) * sp.S : tiles;
+  const int grid = tiles * sp.S;
   note_kernel(dma_kernel_name<BM, BN, WM, WN, NS, SCH, SPS, false, Desc>());
   note_dims(M, N, bd.K, dims_flags);
   launch((dma_gemm_kernel<BM, BN, WM, WN, NS, SCH, SPS, false, Desc>), dim3(grid), dim3(NT), 0,
@@ -1830,6 +1825,75 @@ static inline long long ceil_div(long long a, long long b) { return (a + b - 1) 
 
 // Tile-shape override for tuning sweeps (0 = automatic choice).
 static thread_local int g_forced_tile = 0;
+
+// Tile and split choice.  A launch's time is modelled as
+//   3 + rounds * (fix + slices * per_slice) + (splits > 1 ? split0 + splits * split1 : 0)   [us]
+// with rounds = ceil(tiles * splits / slots), slots = workgroups the chip holds
+// at a time, slices = 64-deep K slices of one split.  The constants are fits to
+// launches timed alone (graph replays, fp16 N(0,1) data) over 45 linears and
+// convs of 144-16384 rows, 320-10240 columns and K = 640-23040: the modelled
+// choice was the fastest of seven tiles and seven split counts or within 8% of
+// it everywhere.  Before, the choice followed the shapes of one image size;
+// others fell on partly empty grids, and below 128 tiles on a register-staged
+// kernel without splits (us, before -> after):
+//   conv 480x640x5760 51.7 -> 20.4      conv 240x1280x11520 95 -> 27
+//   conv 510x1280x11520 93 -> 33        conv 768x1280x23040 179 -> 65
+//   conv 15840x320x2880 59 -> 40        conv 8512x320x2880 53 -> 31
+//   conv 2048x1280x17280 113 -> 99      linear 270x1280x5120 31.5 -> 20.4
+//   linear 2448x640x640 12.1 -> 9.1     linear 988x1280x1280 16.4 -> 12.5
+struct TileCost {
+  int id, bm, bn, slots;
+  float fix, per_slice, per_slice_conv;
+  float split0, split1;  // split0 < 0: never split
+};
+// id as in dlm_gemm_force_tile
+constexpr TileCost kTiles[] = {
+    {45, 256, 160, 256, 9.0f, 1.06f, 1.13f, 18.0f, 1.0f},  {24, 128, 160, 256, 5.0f, 0.72f, 0.72f, 6.0f, 0.5f},
+    {14, 128, 128, 256, 2.5f, 0.60f, 0.60f, 5.0f, 0.7f},   {11, 128, 64, 256, 2.5f, 0.34f, 0.45f, 4.5f, 0.9f},
+    {35, 128, 80, 256, 3.4f, 0.435f, 0.54f, 5.0f, 0.8f},   {29, 128, 128, 512, 3.0f, 1.2f, 1.13f, -1.0f, 0.0f},
+    {19, 256, 128, 256, 7.0f, 0.95f, 0.95f, -1.0f, 0.0f},
+};
+// LayerNorm-folding forms (never split: the row statistics would need a
+// merge of their own)
+constexpr TileCost kLnTiles[] = {
+    {41, 256, 160, 256, 9.0f, 1.2f, 1.2f, -1.0f, 0.0f},  {24, 128, 160, 256, 5.0f, 0.95f, 0.95f, -1.0f, 0.0f},
+    {14, 128, 128, 256, 2.5f, 0.75f, 0.75f, -1.0f, 0.0f}, {11, 128, 64, 256, 2.5f, 0.45f, 0.45f, -1.0f, 0.0f},
+    {35, 128, 80, 256, 3.4f, 0.45f, 0.45f, -1.0f, 0.0f},  {40, 128, 128, 512, 3.0f, 1.35f, 1.35f, -1.0f, 0.0f},
+};
+constexpr int kMaxSplits = 12;
+struct GemmPlan {
+  int tile, splits;
+};
+template <size_t NT>
+static GemmPlan plan_gemm(const TileCost (&tiles)[NT], int M, int N, int nk, bool conv, bool geglu, int max_splits) {
+  GemmPlan best{29, 1};
+  float best_t = 3e38f;
+  for (const TileCost& t : tiles) {
+    const long long grid = ceil_div(M, t.bm) * ceil_div(N, t.bn);
+    // two workgroups to a CU only pay where both have a tile; 256x128 only for
+    // convs of up to four 128x128 tiles per CU (larger grids keep 128x128,
+    // whose fp32 epilogues pass under the other workgroup's main loop: VAE
+    // decode 17.0 against 17.4 ms)
+    if (t.slots == 512 && grid < 256) continue;
+    if (t.id == 19 && (!conv || ceil_div(M, 128) * ceil_div(N, 128) >= 4 * 256)) continue;
+    for (int S = 1; S <= max_splits && S <= nk; ++S) {
+      if (S > 1 && (t.split0 < 0.0f || (size_t)grid * S * t.bm * t.bn > kSplitWsFloats || grid > kSplitCounters)) break;
+      const int kps = (nk + S - 1) / S;
+      if ((nk + kps - 1) / kps != S) continue;  // the same splits as a smaller S
+      // a last round with one workgroup to a CU instead of two runs faster
+      float rounds = (float)ceil_div(grid * S, t.slots);
+      if (t.slots == 512 && grid % 512 >= 1 && grid % 512 <= 256) rounds -= 0.4f;
+      const float fix = t.fix + (geglu && t.slots == 512 ? 2.5f : 0.0f);
+      const float us = rounds * (fix + (float)kps * (conv ? t.per_slice_conv : t.per_slice)) +
+                       (S > 1 ? t.split0 + (float)S * t.split1 : 0.0f);
+      if (us < best_t) {
+        best_t = us;
+        best = GemmPlan{t.id, S};
+      }
+    }
+  }
+  return best;
+}
 
 static bool al8(const void* p) { return ((uintptr_t)p & 7) == 0; }
 
@@ -1891,13 +1955,13 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
     return fail(DLM_ERR_UNSUPPORTED, "fp32 output/residual with a GEGLU or V^T epilogue");
   const bool dma = dma_epilogue_ok(ep) && dma_operand_ok(ad) && dma_operand_ok(bd);
   if (ep.ln_c1) {
-    // LayerNorm-folding linears: the tiles of the plain heuristic below for the
-    // UNet's shapes, 128x128 prefetch tiles for any other
     if constexpr (!std::is_same<Desc, RowDesc>::value) {
       return fail(DLM_ERR_UNSUPPORTED, "LayerNorm folding applies to linears only");
     } else {
       if (!dma) return fail(DLM_ERR_UNSUPPORTED, "LayerNorm-folding GEMM needs aligned operands");
       switch (g_forced_tile) {  // tuning aid: the tiles with a folding kernel
+        case 11: return launch_dma<128, 64, 64, 32, 4>(ad, bd, ep, M, N, s);
+        case 14: return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s);
         case 24: return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
         case 28: return launch_dma<256, 160, 64, 80, 3, kPrefetch>(ad, bd, ep, M, N, s);
         case 29: return launch_dma<128, 128, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s);
@@ -1909,23 +1973,15 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
         case 0: break;
         default: return fail(DLM_ERR_UNSUPPORTED, "forced tile has no LayerNorm-folding kernel");
       }
-      // Every wave accumulates the statistics of its own rows, so waves that
-      // hold fewer row blocks (and fewer waves sharing rows) spend less VALU
-      // on them.  Measured against LayerNorm + linear, graph-replayed (us):
-      // QKV 2048x3840x1280 128x128 (32x64 waves) 35.4 vs 43.5; cross Q
-      // 2048x1280x1280 128x80 15.7 vs 23.5; GEGLU 2048x10240x1280 256x160
-      // (32x160 waves) 79.9 vs 86.7; 8192 rows: QKV 41.3 vs 45.7, Q 18.0 vs
-      // 26.4, GEGLU 99.4 vs 100.3.
-      const long long t256 = ceil_div(M, 256) * (N / 160), t80 = ceil_div(M, 128) * (N / 80);
-      const long long t160 = ceil_div(M, 128) * (N / 160);
-      const int nk = (int)ceil_div(bd.K, BK);
-      if (ep.act == DLM_ACT_GEGLU && N % 160 == 0 && t256 >= kCUs)
-        return launch_dma<256, 160, 32, 160, 3, kPrefetch>(ad, bd, ep, M, N, s);
-      if (!ep.vt && ep.act != DLM_ACT_GEGLU && N % 80 == 0 && t80 >= kCUs * 3 / 4 && t80 <= kCUs)
-        return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
-      if (!ep.vt && ep.act != DLM_ACT_GEGLU && N % 160 == 0 && N <= 1280 && t160 >= kCUs && nk <= 100)
-        return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
-      return launch_dma<128, 128, 32, 64, 2, kPrefetch>(ad, bd, ep, M, N, s);
+      const GemmPlan pl = plan_gemm(kLnTiles, M, N, (int)ceil_div(bd.K, BK), false, ep.act == DLM_ACT_GEGLU, 1);
+      switch (pl.tile) {
+        case 11: return launch_dma<128, 64, 64, 32, 4>(ad, bd, ep, M, N, s);
+        case 14: return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s);
+        case 24: return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
+        case 35: return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
+        case 41: return launch_dma<256, 160, 32, 160, 3, kPrefetch>(ad, bd, ep, M, N, s);
+        default: return launch_dma<128, 128, 32, 64, 2, kPrefetch>(ad, bd, ep, M, N, s);
+      }
     }
   }
   if (dma) {
@@ -1976,83 +2032,28 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
       // tile that is mostly padding
       if (N <= 16 && !ep.vt && ep.act != DLM_ACT_GEGLU && ceil_div(M, 128) >= kCUs / 2)
         return launch_dma<128, 16, 16, 16, 3>(ad, bd, ep, M, N, s);
-      // Measured on the UNet's shapes (warmed-up clocks, N(0,1) data):
-      // 8-wave tiles (two waves per SIMD) everywhere.  128x128 tiles: two
-      // slices in flight when two workgroups share a CU, four when the grid
-      // leaves CUs with one.  GEGLU can take any tile (its value/gate pairs
-      // sit in lanes 16 apart, so any 16-column-multiple wave works).
-      const long long t128 = ceil_div(M, 128) * ceil_div(N, 128);
-      const bool pf = !(g_variant & 2);
-      // GEGLU with at least one 256x160 tile per CU: those, in ping-pong
-      // (2048x10240x1280 71 -> 65 us, 8192x5120x640 89 -> 79 us against
-      // the 128x128 prefetch tiles it took before).
-      if (ep.act == DLM_ACT_GEGLU && N % 160 == 0 && ceil_div(M, 256) * (N / 160) >= kCUs)
-        return pf ? launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s)
-                  : launch_dma<256, 160, 64, 80, 3>(ad, bd, ep, M, N, s);
-      // Output widths that are multiples of 160 (SDXL's 320 / 640 / 1280
-      // channels): 160-column tiles give whole waves of tiles on 256 CUs
-      // where 128-column tiles leave a partial wave; few tiles with a long K
-      // are split-K so every CU gets work.  Choices measured per UNet level
-      // (B=2): 32768x320 convs 256x160 (four splits from 80 slices on measured
-      // the same as none; 8192x1280x11520 is ~130 us faster unsplit), 8192
-      // rows 128x160 up to 100 slices and 256x160 x2 splits beyond, 2048 rows
-      // 128x160 x2 splits from 44 slices, 256x160 x4 from 300.  Two splits of
-      // a grid that already fills the chip measured slower than one or four.
-      const int nk = (int)ceil_div(bd.K, BK);
-      // 2048-row outputs 1280 wide (one 1024-token level at B=2) and the
-      // 8192x320 stride-2 conv: 128x80 tiles, 8 waves of 16x80 -> exactly
-      // 256 tiles.  Ring of three two-slice stages (one barrier per 128 of
-      // K): 15.5 / 40.3 us at K = 1280 / 5120 against 16.4 / 42.6 for a
-      // five-slice ring and 16.2 / 43.9 for 128x128; the conv 39.1 us
-      // against 47.3 for 128x160 x2 splits.  Convolutions with a long K
-      // (2048x1280x11520) stay on split 128x160 tiles.
-      if ((std::is_same<Desc, RowDesc>::value || nk <= 100) && !ep.vt && N % 80 == 0 &&
-          ceil_div(M, 128) * (N / 80) >= kCUs * 3 / 4 &&
-          ceil_div(M, 128) * (N / 80) <= kCUs && !(g_variant & 1))
-        return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
-      if (!ep.vt && N % 160 == 0 && N <= 1280 && !(g_variant & 1)) {
-        const long long t256 = ceil_div(M, 256) * (N / 160), t160 = ceil_div(M, 128) * (N / 160);
-        if (t256 >= kCUs)
-          return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, !pf && nk >= 80 ? 4 : 1);
-        if (t160 >= kCUs) {
-          if (nk <= 100) return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s);
-          return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, 2);
-        } else if (nk >= 300 && t256 * 4 >= kCUs) {
-          return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, 4);
-        } else if (nk >= 44 && t160 * 4 >= kCUs) {
-          return launch_dma<128, 160, 32, 80, 3>(ad, bd, ep, M, N, s, t160 * 2 >= kCUs ? 2 : 4);
-        }
-      }
       // Outputs of 129-192 rows with at least one 160-column tile per CU (the
       // text tokens' K/V projection of every transformer block at CFG batch
       // 2, 154 x 166400 x 2048): 192x160 tiles (8 waves of 48x80) compute the
       // rows as 192 instead of 256, 235-251 -> 206-212 us per launch,
       // bit-identical.
-      if (std::is_same<Desc, RowDesc>::value && M > 128 && M <= 192 && N % 160 == 0 && N / 160 >= kCUs &&
+      if (std::is_same<Desc, ConvDesc>::value == false && M > 128 && M <= 192 && N % 160 == 0 && N / 160 >= kCUs &&
           ep.act != DLM_ACT_GEGLU)
         return launch_dma<192, 160, 48, 80, 3>(ad, bd, ep, M, N, s);
-      if (t128 >= kCUs / 2) {
-        if (N % 128 != 0)
-          return ceil_div(M, 128) * ceil_div(N, 64) >= kCUs
-                     ? launch_dma<128, 64, 64, 32, 2>(ad, bd, ep, M, N, s)
-                     : launch_dma<128, 64, 64, 32, 4>(ad, bd, ep, M, N, s);
-        // convolutions with one to four 128x128 tiles per CU: 256x128 tiles
-        // (fewer operand bytes per MFMA).  Larger grids keep 128x128, two
-        // workgroups to a CU, whose epilogues pass under each other's main
-        // loops (the VAE's 3x3 convs: 256x128 tiles 17.0 -> 17.4 ms a decode,
-        // although 4% faster on their own without the fp32 epilogue).
-        if (std::is_same<Desc, ConvDesc>::value && t128 >= kCUs && t128 < 4 * kCUs)
-          return launch_dma<256, 128, 64, 64, 3>(ad, bd, ep, M, N, s);
-        // one workgroup's ring of two slices: the prefetch form (2048x3840x1280
-        // QKV ~2 us faster per launch, 8192x1920x640 the same)
-        if (t128 >= kCUs)
-          return pf ? launch_dma<128, 128, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s)
-                    : launch_dma<128, 128, 64, 32, 2>(ad, bd, ep, M, N, s);
-        return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s);
+      constexpr bool conv = std::is_same<Desc, ConvDesc>::value;
+      const int nk = (int)ceil_div(bd.K, BK);
+      GemmPlan pl = plan_gemm(kTiles, M, N, nk, conv, ep.act == DLM_ACT_GEGLU, t_no_split || (g_variant & 1) ? 1 : kMaxSplits);
+      // no workspace (a stream that met capture first, memory): plan without splits
+      if (pl.splits > 1 && !split_workspace(s)) pl = plan_gemm(kTiles, M, N, nk, conv, ep.act == DLM_ACT_GEGLU, 1);
+      switch (pl.tile) {
+        case 11: return launch_dma<128, 64, 64, 32, 4>(ad, bd, ep, M, N, s, pl.splits);
+        case 14: return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s, pl.splits);
+        case 19: return launch_dma<256, 128, 64, 64, 3>(ad, bd, ep, M, N, s);
+        case 24: return launch_dma<128, 160, 32, 80, 4>(ad, bd, ep, M, N, s, pl.splits);
+        case 29: return launch_dma<128, 128, 64, 32, 2, kPrefetch>(ad, bd, ep, M, N, s);
+        case 35: return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s, pl.splits);
+        default: return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s, pl.splits);
       }
-      if (ep.vt)  // the transposed-V epilogue exists only in the DMA core
-        return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s);
-      // fewer than 128 tiles of 128x128: the small-tile kernel below
     }
   }
   if (ep.vt) return fail(DLM_ERR_UNSUPPORTED, "transposed-V output needs aligned operands");

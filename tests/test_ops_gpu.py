@@ -185,6 +185,34 @@ def test_conv_nhwc_concat_shortcut_residual_tbias(gpu):
     assert_close(ops.nhwc_to_nchw(y), ref, "conv+shortcut+tbias")
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 320, 640), (63, 1284, 5128), (144, 1280, 5120), (257, 640, 2560),
+                                   (532, 1280, 5120), (1224, 640, 2568)])
+def test_linear_planned_splits(gpu, M, N, K):
+    """Grids that leave CUs idle take small tiles and split-K: partial tiles, a K tail that ends inside
+    the last split, and the same result on every launch."""
+    announce(f"linear planned splits {M}x{N}x{K}")
+    x, w, b, r = randn((M, K), 120), randn((N, K), 121, std=K ** -0.5), randn((N,), 122), randn((M, N), 123)
+    args = dict(bias=to_gpu(b), residual=to_gpu(r))
+    y = ops.linear(to_gpu(x), to_gpu(w), **args)
+    # fp32 sums in another order and one fp16 rounding (2^-11 of the value)
+    ref = x @ w.t() + b + r
+    assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
+    assert torch.equal(y, ops.linear(to_gpu(x), to_gpu(w), **args))
+
+
+@pytest.mark.parametrize("B,H,W,Ci,Co,stride,up", [(1, 1, 1, 640, 1280, 1, False), (1, 12, 20, 1280, 1280, 1, False),
+                                                   (2, 15, 17, 640, 320, 2, False), (1, 9, 7, 640, 640, 1, True),
+                                                   (2, 16, 8, 320, 1280, 1, False)])
+def test_conv_planned_splits(gpu, B, H, W, Ci, Co, stride, up):
+    """The same for 3x3 convs: one pixel, odd sizes, strides, upsampling."""
+    announce(f"conv planned splits {B}x{H}x{W} {Ci}-{Co} s{stride} up{up}")
+    x, w, b = randn((B, Ci, H, W), 124), randn((Co, Ci, 3, 3), 125, std=(9 * Ci) ** -0.5), randn((Co,), 126)
+    y = ops.nhwc_to_nchw(ops.conv2d_nhwc(ops.nchw_to_nhwc(to_gpu(x)), ops.pack_conv_weight(to_gpu(w)), KH=3, KW=3,
+                                         stride=stride, pad=1, bias=to_gpu(b), upsample=up))
+    ref = torch.nn.functional.conv2d(R.upsample_nearest2x(x) if up else x, w, b, stride=stride, padding=1)
+    assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
+
+
 def test_conv_nhwc_concat_upsample_residual(gpu):
     N, H, W, Ca, Cb, Cout = 2, 8, 12, 64, 128, 64
     announce("conv nhwc concat input + nearest2x upsample + residual")
