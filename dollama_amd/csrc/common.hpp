@@ -164,6 +164,36 @@ __device__ __forceinline__ float2 gn_stat_finish(float s1, float s2, float shift
   return make_float2(shift + md, fmaxf(__builtin_fmaf(-s1, md, s2), 0.0f));
 }
 
+// dst[c][r] = src[r][c] of one 64 x 64 block at (r0, c0), for c < cols and
+// r < ld_out (zero for r >= rows).  256 threads; a thread reads 8 columns of
+// two rows, packs each column's pair of halfs into a dword for LDS (row
+// stride 33 dwords: the 64 lanes of a write hit 64 banks), and writes 8 rows
+// of a column: every access to memory is 16 bytes.  Needs cols, ld_src and
+// ld_out multiples of 8 and 16-byte aligned src and dst.
+__device__ __forceinline__ void transpose_tile64(const f16* __restrict__ src, int rows, int cols, int ld_src,
+                                                 f16* __restrict__ dst, int ld_out, int r0, int c0,
+                                                 uint32_t* tile) {
+  const int t = threadIdx.x, pair = t >> 3, ch = t & 7;
+  f16x8 a{}, b{};
+  if (c0 + ch * 8 < cols) {
+    const f16* p = src + (size_t)(r0 + 2 * pair) * ld_src + c0 + ch * 8;
+    if (r0 + 2 * pair < rows) a = *reinterpret_cast<const f16x8*>(p);
+    if (r0 + 2 * pair + 1 < rows) b = *reinterpret_cast<const f16x8*>(p + ld_src);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) tile[(ch * 8 + j) * 33 + pair] = __builtin_bit_cast(uint32_t, f16x2{a[j], b[j]});
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int c = pair + 32 * s;
+    u32x4 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = tile[c * 33 + ch * 4 + q];
+    if (c0 + c < cols && r0 + ch * 8 < ld_out)
+      *reinterpret_cast<u32x4*>(dst + (size_t)(c0 + c) * ld_out + r0 + ch * 8) = v;
+  }
+}
+
 // Grid of a grid-stride elementwise launch over n items.
 static inline int grid_for(long long n, int threads = 256, int cap = 8192) {
   return (int)std::max<long long>(1, std::min<long long>((n + threads - 1) / threads, cap));
