@@ -213,6 +213,33 @@ def test_conv_planned_splits(gpu, B, H, W, Ci, Co, stride, up):
     assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
 
 
+@pytest.mark.parametrize("B,S,N,col0,K,ld", [(2, 77, 2560, 1280, 256, 80), (3, 12, 320, 160, 64, 16),
+                                             (1, 1024, 1920, 1280, 64, 1024), (2, 100, 300, 100, 72, 104),
+                                             (2, 988, 640, 320, 128, 992), (1, 131, 512, 128, 64, 133)])
+def test_linear_vt_tiles(gpu, B, S, N, col0, K, ld):
+    """The transposed-V output by whole tiles: token counts that are and are not multiples of 4, a
+    column split inside a tile, partial row and column tiles, and the zero padding of every V^T row."""
+    announce(f"linear_vt B={B} S={S} N={N} col0={col0} K={K} ld={ld}")
+    x, w = randn((B * S, K), 127), randn((N, K), 128, std=K ** -0.5)
+    y, vt = ops.linear_vt(to_gpu(x), to_gpu(w), col0, S, vt_ld=ld)
+    ref = x @ w.t()
+    assert_close(y[:, :col0], ref[:, :col0], "columns before V", rel_tol=5e-4)
+    got = from_gpu(vt).reshape(B, N - col0, ld)
+    assert_close(got[:, :, :S], ref[:, col0:].reshape(B, S, N - col0).transpose(1, 2), "V^T", rel_tol=5e-4)
+    assert not got[:, :, S:].any()
+
+
+@pytest.mark.parametrize("N,C,H,W,cp", [(1, 4, 8, 9, 64), (2, 320, 5, 8, 320), (1, 65, 8, 8, 72), (2, 8, 1, 8, 8),
+                                        (1, 72, 13, 16, 72), (1, 64, 7, 9, 64)])
+def test_layout_transposes(gpu, N, C, H, W, cp):
+    """NCHW <-> channels-last: partial tiles, channel padding, and rows that are no whole vectors."""
+    announce(f"transposes {N}x{C}x{H}x{W} pad {cp}")
+    x = to_gpu(randn((N, C, H, W), 129))
+    y = ops.nchw_to_nhwc(x, cp)
+    assert torch.equal(y[..., :C], x.permute(0, 2, 3, 1)) and not y[..., C:].any()
+    assert torch.equal(ops.nhwc_to_nchw(y, C), x)
+
+
 def test_conv_nhwc_concat_upsample_residual(gpu):
     N, H, W, Ca, Cb, Cout = 2, 8, 12, 64, 128, 64
     announce("conv nhwc concat input + nearest2x upsample + residual")
