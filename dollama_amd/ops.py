@@ -43,8 +43,17 @@ def stream_handle() -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+# What every launch passes, as plain integers: the bindings declare c_void_p
+# arguments and fields, which take them, and neither a Stream object nor a
+# c_void_p per pointer has to be built (a call of five small launches was bound
+# by this file: 46 -> 33 us).
+def _stream() -> int:
+    """Handle of the current device's current stream."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def _p(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _need(t: Optional[torch.Tensor], numel: int, name: str, dtype=torch.float16, optional=False):
@@ -83,7 +92,7 @@ def launch_conv2d(d_in, d_weight, d_bias, d_out, N, Cin, H, W, Cout, KH, KW,
     _need(d_bias, Cout, "d_bias", optional=True)
     _need(d_out, N * Cout * Ho * Wo, "d_out")
     call("dlm_conv2d_fp16", _p(d_in), _p(d_weight), _p(d_bias), _p(d_out), N, Cin, H, W, Cout,
-         KH, KW, stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w, stream_handle())
+         KH, KW, stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w, _stream())
 
 
 def launch_gemm_fp16(d_A, d_B, d_C, M, N, K, alpha=1.0, beta=0.0, transA=False, transB=False):
@@ -94,7 +103,7 @@ def launch_gemm_fp16(d_A, d_B, d_C, M, N, K, alpha=1.0, beta=0.0, transA=False, 
     _need(d_B, K * N, "d_B")
     _need(d_C, M * N, "d_C")
     call("dlm_gemm_fp16", _p(d_A), _p(d_B), _p(d_C), M, N, K, float(alpha), float(beta),
-         int(bool(transA)), int(bool(transB)), stream_handle())
+         int(bool(transA)), int(bool(transB)), _stream())
 
 
 def _gn(d_in, d_gamma, d_beta, d_out, N, C, H, W, num_groups, eps, silu):
@@ -105,7 +114,7 @@ def _gn(d_in, d_gamma, d_beta, d_out, N, C, H, W, num_groups, eps, silu):
     _need(d_gamma, C, "d_gamma", optional=True)
     _need(d_beta, C, "d_beta", optional=True)
     call("dlm_group_norm_fp16", _p(d_in), _p(d_gamma), _p(d_beta), _p(d_out), N, C, H, W,
-         num_groups, float(eps), int(silu), stream_handle())
+         num_groups, float(eps), int(silu), _stream())
 
 
 def launch_group_norm(d_in, d_gamma, d_beta, d_out, N, C, H, W, num_groups, eps):
@@ -132,7 +141,7 @@ def launch_layer_norm(d_in, d_gamma, d_beta, d_out, rows, C, eps=1e-5):
     _need(d_gamma, C, "d_gamma", optional=True)
     _need(d_beta, C, "d_beta", optional=True)
     call("dlm_layer_norm_fp16", _p(d_in), _p(d_gamma), _p(d_beta), _p(d_out), rows, C,
-         float(eps), stream_handle())
+         float(eps), _stream())
 
 
 def launch_attention(d_q, d_k, d_v, d_out, B, H, Sq, Sk, Dh, scale):
@@ -144,7 +153,7 @@ def launch_attention(d_q, d_k, d_v, d_out, B, H, Sq, Sk, Dh, scale):
     _need(d_v, B * H * Sk * Dh, "d_v")
     _need(d_out, B * H * Sq * Dh, "d_out")
     call("dlm_attention_fp16", _p(d_q), _p(d_k), _p(d_v), _p(d_out), B, H, Sq, Sk, Dh,
-         float(scale), stream_handle())
+         float(scale), _stream())
 
 
 launch_attention_fast = launch_attention
@@ -156,7 +165,7 @@ def launch_geglu(d_in, d_out, tokens, d):
         return
     _need(d_in, tokens * 2 * d, "d_in")
     _need(d_out, tokens * d, "d_out")
-    call("dlm_geglu_fp16", _p(d_in), _p(d_out), tokens, d, stream_handle())
+    call("dlm_geglu_fp16", _p(d_in), _p(d_out), tokens, d, _stream())
 
 
 def _unary(name, d_in, d_out, n):
@@ -164,7 +173,7 @@ def _unary(name, d_in, d_out, n):
         return
     _need(d_in, n, "d_in")
     _need(d_out, n, "d_out")
-    call(name, _p(d_in), _p(d_out), n, stream_handle())
+    call(name, _p(d_in), _p(d_out), n, _stream())
 
 
 def launch_silu(d_in, d_out, n):
@@ -189,7 +198,7 @@ def launch_add(d_a, d_b, d_out, n):
     _need(d_a, n, "d_a")
     _need(d_b, n, "d_b")
     _need(d_out, n, "d_out")
-    call("dlm_add_fp16", _p(d_a), _p(d_b), _p(d_out), n, stream_handle())
+    call("dlm_add_fp16", _p(d_a), _p(d_b), _p(d_out), n, _stream())
 
 
 def launch_upsample_nearest2x(d_in, d_out, N, C, H, W):
@@ -198,7 +207,7 @@ def launch_upsample_nearest2x(d_in, d_out, N, C, H, W):
         return
     _need(d_in, N * C * H * W, "d_in")
     _need(d_out, N * C * 4 * H * W, "d_out")
-    call("dlm_upsample_nearest2x_fp16", _p(d_in), _p(d_out), N, C, H, W, stream_handle())
+    call("dlm_upsample_nearest2x_fp16", _p(d_in), _p(d_out), N, C, H, W, _stream())
 
 
 def launch_bias_add_rowvec(d_in, d_bias, d_out, tokens, C):
@@ -208,7 +217,7 @@ def launch_bias_add_rowvec(d_in, d_bias, d_out, tokens, C):
     _need(d_in, tokens * C, "d_in")
     _need(d_bias, C, "d_bias")
     _need(d_out, tokens * C, "d_out")
-    call("dlm_bias_add_rowvec_fp16", _p(d_in), _p(d_bias), _p(d_out), tokens, C, stream_handle())
+    call("dlm_bias_add_rowvec_fp16", _p(d_in), _p(d_bias), _p(d_out), tokens, C, _stream())
 
 
 def launch_bias_add_channel(d_in, d_bias, d_out, N, C, H, W):
@@ -219,7 +228,7 @@ def launch_bias_add_channel(d_in, d_bias, d_out, N, C, H, W):
     _need(d_bias, C, "d_bias")
     _need(d_out, N * C * H * W, "d_out")
     call("dlm_bias_add_channel_fp16", _p(d_in), _p(d_bias), _p(d_out), N, C, H, W,
-         stream_handle())
+         _stream())
 
 
 def launch_conv_bias_biasch(d_conv, d_convbias, d_tproj, d_out, B, Cout, H, W):
@@ -231,7 +240,7 @@ def launch_conv_bias_biasch(d_conv, d_convbias, d_tproj, d_out, B, Cout, H, W):
     _need(d_tproj, B * Cout, "d_tproj")
     _need(d_out, B * Cout * H * W, "d_out")
     call("dlm_conv_bias_biasch_fp16", _p(d_conv), _p(d_convbias), _p(d_tproj), _p(d_out), B, Cout,
-         H, W, stream_handle())
+         H, W, _stream())
 
 
 def launch_conv_bias_residual(d_conv, d_convbias, d_residual, d_out, B, Cout, H, W):
@@ -243,7 +252,7 @@ def launch_conv_bias_residual(d_conv, d_convbias, d_residual, d_out, B, Cout, H,
     _need(d_residual, B * Cout * H * W, "d_residual")
     _need(d_out, B * Cout * H * W, "d_out")
     call("dlm_conv_bias_residual_fp16", _p(d_conv), _p(d_convbias), _p(d_residual), _p(d_out), B,
-         Cout, H, W, stream_handle())
+         Cout, H, W, _stream())
 
 
 def launch_timestep_embedding(d_out, timestep, dim, max_period=10000.0):
@@ -252,7 +261,7 @@ def launch_timestep_embedding(d_out, timestep, dim, max_period=10000.0):
         return
     _need(d_out, (dim // 2) * 2, "d_out")
     call("dlm_timestep_embedding_fp16", _p(d_out), float(timestep), dim, float(max_period),
-         stream_handle())
+         _stream())
 
 
 # ---------------------------------------------------------------------------
@@ -282,10 +291,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None, residual=None, act=ACT_N
             raise ValueError("gn_stats needs M = samples x tokens")
         _need(gn_stats, group_norm_workspace_bytes(M // tokens, N, tokens), "gn_stats", dtype=torch.uint8)
         call("dlm_linear_gn_stats_fp16", _p(x), K, _p(w), K, _p(bias), _p(residual), ncols, _p(out), ncols,
-             M, N, K, float(alpha), float(beta), int(act), int(tokens), _p(gn_stats), stream_handle())
+             M, N, K, float(alpha), float(beta), int(act), int(tokens), _p(gn_stats), _stream())
         return out
     call("dlm_linear_fp16", _p(x), K, _p(w), K, _p(bias), _p(residual), ncols, _p(out), ncols,
-         M, N, K, float(alpha), float(beta), int(act), stream_handle())
+         M, N, K, float(alpha), float(beta), int(act), _stream())
     return out
 
 
@@ -305,7 +314,7 @@ def linear_f32out(x: torch.Tensor, w: torch.Tensor, bias=None, residual=None, ac
     _need(residual, M * N, "residual", optional=True, dtype=torch.float32)
     _need(out, M * N, "out", dtype=torch.float32)
     call("dlm_linear_f32out_fp16", _p(x), K, _p(w), K, _p(bias), _p(residual), N, _p(out), N,
-         M, N, K, float(alpha), float(beta), int(act), stream_handle())
+         M, N, K, float(alpha), float(beta), int(act), _stream())
     return out
 
 
@@ -316,7 +325,7 @@ def softmax_rows(s: torch.Tensor, out=None) -> torch.Tensor:
         out = torch.empty(rows, cols, dtype=torch.float16, device=s.device)
     _need(s, rows * cols, "s", dtype=torch.float32)
     _need(out, rows * cols, "out")
-    call("dlm_softmax_rows_f32_fp16", _p(s), cols, _p(out), cols, rows, cols, stream_handle())
+    call("dlm_softmax_rows_f32_fp16", _p(s), cols, _p(out), cols, rows, cols, _stream())
     return out
 
 
@@ -324,7 +333,7 @@ def cast_f32_to_f16(x: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
     """fp16(x * scale)."""
     _need(x, x.numel(), "x", dtype=torch.float32)
     out = torch.empty(x.shape, dtype=torch.float16, device=x.device)
-    call("dlm_cast_f32_to_f16", _p(x), _p(out), x.numel(), float(scale), stream_handle())
+    call("dlm_cast_f32_to_f16", _p(x), _p(out), x.numel(), float(scale), _stream())
     return out
 
 
@@ -343,7 +352,7 @@ def linear_vt(x: torch.Tensor, w: torch.Tensor, vt_col0: int, tokens: int, bias=
     _need(w, N * K, "w")
     _need(bias, N, "bias", optional=True)
     call("dlm_linear_vt_fp16", _p(x), K, _p(w), K, _p(bias), _p(y), vt_col0, _p(vt), vt_col0,
-         tokens, vt_ld, M, N, K, stream_handle())
+         tokens, vt_ld, M, N, K, _stream())
     return y, vt
 
 
@@ -359,7 +368,7 @@ def ln_fold(w: torch.Tensor, gamma=None, beta=None, bias=None):
     _need(beta, K, "beta", optional=True)
     _need(bias, N, "bias", optional=True)
     call("dlm_ln_fold_fp16", _p(w), K, N, K, _p(gamma), _p(beta), _p(bias), _p(wo), K, _p(c1),
-         _p(c2), stream_handle())
+         _p(c2), _stream())
     return wo, c1, c2
 
 
@@ -379,7 +388,7 @@ def linear_ln(x: torch.Tensor, w_folded, c1, c2, eps: float, residual=None, act=
     _need(residual, M * ncols, "residual", optional=True)
     _need(out, M * ncols, "out")
     call("dlm_linear_ln_fp16", _p(x), K, _p(w_folded), K, _p(c1), _p(c2), float(eps), _p(residual),
-         ncols, _p(out), ncols, M, N, K, float(beta), int(act), stream_handle())
+         ncols, _p(out), ncols, M, N, K, float(beta), int(act), _stream())
     return out
 
 
@@ -396,7 +405,7 @@ def linear_vt_ln(x: torch.Tensor, w_folded, c1, c2, eps: float, vt_col0: int, to
     _need(c1, N, "c1", dtype=torch.float32)
     _need(c2, N, "c2", dtype=torch.float32)
     call("dlm_linear_vt_ln_fp16", _p(x), K, _p(w_folded), K, _p(c1), _p(c2), float(eps), _p(y),
-         vt_col0, _p(vt), vt_col0, tokens, vt_ld, M, N, K, stream_handle())
+         vt_col0, _p(vt), vt_col0, tokens, vt_ld, M, N, K, _stream())
     return y, vt
 
 
@@ -408,7 +417,7 @@ def pack_geglu(w: torch.Tensor, b: Optional[torch.Tensor]):
     bo = None if b is None else torch.empty_like(b)
     _need(w, two_d * K, "w")
     _need(b, two_d, "b", optional=True)
-    call("dlm_geglu_pack_fp16", _p(w), _p(b), _p(wo), _p(bo), d, K, stream_handle())
+    call("dlm_geglu_pack_fp16", _p(w), _p(b), _p(wo), _p(bo), d, K, _stream())
     return wo, bo
 
 
@@ -423,7 +432,7 @@ def pack_conv_weight(w: torch.Tensor, cin_pad: Optional[int] = None, out=None, l
     _need(w, w.numel(), "w")
     _need(out, Cout * ld, "out")
     call("dlm_conv_weight_pack_fp16", _p(w), _p(out), Cout, Cin, KH, KW, cp, ld, col0,
-         stream_handle())
+         _stream())
     return out
 
 
@@ -432,7 +441,7 @@ def nchw_to_nhwc(x: torch.Tensor, c_pad: Optional[int] = None) -> torch.Tensor:
     cp = c_pad or C
     out = torch.empty(N, H, W, cp, dtype=torch.float16, device=x.device)
     _need(x, x.numel(), "x")
-    call("dlm_nchw_to_nhwc_fp16", _p(x), _p(out), N, C, H * W, cp, stream_handle())
+    call("dlm_nchw_to_nhwc_fp16", _p(x), _p(out), N, C, H * W, cp, _stream())
     return out
 
 
@@ -441,7 +450,7 @@ def nhwc_to_nchw(x: torch.Tensor, C: Optional[int] = None) -> torch.Tensor:
     C = C or cp
     out = torch.empty(N, C, H, W, dtype=torch.float16, device=x.device)
     _need(x, x.numel(), "x")
-    call("dlm_nhwc_to_nchw_fp16", _p(x), _p(out), N, C, H * W, cp, stream_handle())
+    call("dlm_nhwc_to_nchw_fp16", _p(x), _p(out), N, C, H * W, cp, _stream())
     return out
 
 
@@ -495,7 +504,7 @@ def conv2d_nhwc(x: torch.Tensor, w_packed: torch.Tensor, *, KH: int, KW: int, st
     if gn_stats is not None:
         _need(gn_stats, group_norm_workspace_bytes(N, Cout, Ho * Wo), "gn_stats", dtype=torch.uint8)
     a.gn_stats = _p(gn_stats)
-    call("dlm_conv2d_nhwc_fp16", ctypes.byref(a), stream_handle())
+    call("dlm_conv2d_nhwc_fp16", ctypes.byref(a), _stream())
     return out
 
 
@@ -525,10 +534,10 @@ def group_norm_nhwc(x: torch.Tensor, gamma, beta, groups: int, eps: float, silu:
         if x_b is not None:
             raise ValueError("fp32 GroupNorm takes one source")
         call("dlm_group_norm_nhwc_f32in", _p(x), C, _p(gamma), _p(beta), _p(out), C, N, HW, C,
-             groups, float(eps), int(silu), _p(ws), stream_handle())
+             groups, float(eps), int(silu), _p(ws), _stream())
         return out
     call("dlm_group_norm_nhwc_fp16", _p(x), Ca, Ca, _p(x_b), max(Cb, 8), _p(gamma), _p(beta),
-         _p(out), C, N, HW, C, groups, float(eps), int(silu), _p(ws), stream_handle())
+         _p(out), C, N, HW, C, groups, float(eps), int(silu), _p(ws), _stream())
     return out
 
 
@@ -546,7 +555,7 @@ def group_norm_chunk_stats(x: torch.Tensor, ws: torch.Tensor) -> torch.Tensor:
     N, H, W, C = x.shape
     _need(x, N * H * W * C, "x")
     _need(ws, group_norm_workspace_bytes(N, C, H * W), "ws", dtype=torch.uint8)
-    call("dlm_group_norm_chunk_stats_fp16", _p(x), C, N, H * W, C, _p(ws), stream_handle())
+    call("dlm_group_norm_chunk_stats_fp16", _p(x), C, N, H * W, C, _p(ws), _stream())
     return ws
 
 
@@ -563,7 +572,7 @@ def group_norm_nhwc_prestats(x: torch.Tensor, gamma, beta, groups: int, eps: flo
         out = torch.empty(N, H, W, C, dtype=torch.float16, device=x.device)
     _need(out, N * HW * C, "out")
     call("dlm_group_norm_nhwc_prestats_fp16", _p(x), C, _p(gamma), _p(beta), _p(out), C, N, HW, C,
-         groups, float(eps), int(silu), _p(ws), stream_handle())
+         groups, float(eps), int(silu), _p(ws), _stream())
     return out
 
 
@@ -586,7 +595,7 @@ def group_norm_nhwc_prestats2(x: torch.Tensor, x_b: torch.Tensor, gamma, beta, g
     _need(out, N * HW * C, "out")
     ws = group_norm_workspace(N, C, HW, x.device)
     call("dlm_group_norm_nhwc_prestats2_fp16", _p(x), Ca, Ca, _p(x_b), Cb, _p(ws_a), _p(ws_b), _p(gamma),
-         _p(beta), _p(out), C, N, HW, C, groups, float(eps), int(silu), _p(ws), stream_handle())
+         _p(beta), _p(out), C, N, HW, C, groups, float(eps), int(silu), _p(ws), _stream())
     return out
 
 
@@ -610,7 +619,7 @@ def attention_strided(q, k, v, o, *, B, H, Sq, Sk, q_strides, k_strides, v_strid
     a.v, (a.v_sb, a.v_ss, a.v_sh) = _p(v), v_strides
     a.o, (a.o_sb, a.o_ss, a.o_sh) = _p(o), o_strides
     a.B, a.H, a.Sq, a.Sk, a.Dh, a.scale = B, H, Sq, Sk, Dh, float(scale)
-    call("dlm_attention_strided_fp16", ctypes.byref(a), stream_handle())
+    call("dlm_attention_strided_fp16", ctypes.byref(a), _stream())
     return o
 
 
@@ -638,7 +647,7 @@ def attention_vt(q, k, vt, o, *, B, H, Sq, Sk, q_strides, k_strides, vt_strides,
     a.vt_ld, a.B, a.H, a.Sq, a.Sk, a.scale = vt_ld, B, H, Sq, Sk, float(scale)
     a.k_bytes = k.untyped_storage().nbytes() - k.storage_offset() * 2
     a.vt_bytes = vt.untyped_storage().nbytes() - vt.storage_offset() * 2
-    call("dlm_attention_vt_fp16", ctypes.byref(a), stream_handle())
+    call("dlm_attention_vt_fp16", ctypes.byref(a), _stream())
     return o
 
 
@@ -653,7 +662,7 @@ def linear_small(x, w, bias=None, silu_in=False, act=ACT_NONE, out=None, accumul
     _need(bias, N, "bias", optional=True)
     _need(out, M * N, "out")
     call("dlm_linear_small_fp16", _p(x), K, _p(w), _p(bias), _p(out), N, M, N, K, int(silu_in),
-         int(act), int(accumulate), stream_handle())
+         int(act), int(accumulate), _stream())
     return out
 
 
@@ -667,7 +676,7 @@ def sdxl_embed_inputs(timesteps: torch.Tensor, text_embeds: torch.Tensor, time_i
     t_emb = torch.empty(B, 320, dtype=torch.float16, device=text_embeds.device)
     add_in = torch.empty(B, 2816, dtype=torch.float16, device=text_embeds.device)
     call("dlm_sdxl_embed_inputs_fp16", _p(timesteps), _p(text_embeds), 1280, _p(time_ids), stride,
-         256, _p(t_emb), 320, _p(add_in), B, stream_handle())
+         256, _p(t_emb), 320, _p(add_in), B, _stream())
     return t_emb, add_in
 
 
@@ -682,7 +691,7 @@ def euler_cfg_step(latent: torch.Tensor, noise: torch.Tensor, model_in: torch.Te
     _need(noise, 2 * n, "noise")
     _need(model_in, 2 * n, "model_in")
     call("dlm_euler_cfg_step", _p(latent), _p(noise), _p(model_in), n, float(guidance), float(sigma),
-         float(sigma_next), float(in_scale), stream_handle())
+         float(sigma_next), float(in_scale), _stream())
 
 
 def euler_step(latent: torch.Tensor, noise: torch.Tensor, model_in: torch.Tensor, sigma: float,
@@ -694,7 +703,7 @@ def euler_step(latent: torch.Tensor, noise: torch.Tensor, model_in: torch.Tensor
     _need(noise, n, "noise")
     _need(model_in, n, "model_in")
     call("dlm_euler_step", _p(latent), _p(noise), _p(model_in), n, float(sigma), float(sigma_next),
-         float(in_scale), stream_handle())
+         float(in_scale), _stream())
 
 
 def scale_latent(latent: torch.Tensor, model_in: torch.Tensor, scale: float, copies: int):
@@ -702,4 +711,4 @@ def scale_latent(latent: torch.Tensor, model_in: torch.Tensor, scale: float, cop
     n = latent.numel()
     _need(latent, n, "latent", dtype=torch.float32)
     _need(model_in, copies * n, "model_in")
-    call("dlm_scale_latent_fp16", _p(latent), _p(model_in), n, float(scale), int(copies), stream_handle())
+    call("dlm_scale_latent_fp16", _p(latent), _p(model_in), n, float(scale), int(copies), _stream())
