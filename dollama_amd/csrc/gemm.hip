@@ -24,7 +24,7 @@
 //     phase is conflict-free; the next k-step's fragments are read before
 //     the current k-step's MFMAs.  Optional split-K with a last-arriver
 //     reduction in split order, and an XCD-aware tile order.
-//   - mfma_gemm_kernel (small channel counts, small grids, unaligned
+//   - mfma_gemm_kernel (small channel counts, kernels over 14 taps, unaligned
 //     operands): 4 waves of 32x32x16 MFMA blocks with VGPR-staged,
 //     double-buffered LDS slices (row stride 72 halfs).
 // The A operand is produced by a loader: plain rows for linears, or the
@@ -1784,9 +1784,8 @@ static const char* dma_kernel_name() {
   return n.c_str();
 }
 
-// Tile configurations with a LayerNorm-folding instantiation: the ones the
-// LayerNorm-consuming linears of the UNet take (2048- and 8192-row QKV, cross
-// Q and GEGLU shapes), plus their non-prefetch variants.
+// Tile configurations with a LayerNorm-folding instantiation: those of
+// kLnTiles and their other schedules (dlm_gemm_force_tile).
 template <int BM, int BN, int WM, int WN, int NS, int SCH, int SPS>
 constexpr bool ln_tile() {
   return (BM == 128 && BN == 80 && WM == 16 && WN == 80 && NS == 3 && SCH == kPlain && SPS == 2) ||

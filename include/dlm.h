@@ -180,8 +180,8 @@ int dlm_layer_norm_fp16(const void* in, const void* gamma, const void* beta, voi
 
 /* O = softmax(scale * Q K^T) V, Q/O [B,H,Sq,Dh], K/V [B,H,Sk,Dh], fp32 softmax,
  * any head size (as launch_attention picks a path by Dh,
- * src/kernels/attention.cu:18-21): Dh = 64 runs the flash kernel over a
- * transposed-V copy, other head sizes an fp32 scores GEMM, a row softmax and
+ * src/kernels/attention.cu:18-21): Dh = 40, 64 or 80 runs the flash kernel
+ * over a transposed-V copy, other head sizes an fp32 scores GEMM, a row softmax and
  * a P V^T GEMM in row chunks whose scores stay within 256 MiB.  The copies
  * live in per-stream library staging: not for graph capture.  Replaces
  * launch_attention / launch_attention_fast (src/kernels/attention.cuh:53-73). */
