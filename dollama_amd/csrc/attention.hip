@@ -25,6 +25,7 @@
 // Q, K, V and O are addressed with independent batch / token / head strides,
 // so the fused QKV projection output [B, S, 3C] is read in place.
 #include <algorithm>
+#include <cfloat>
 #include <type_traits>
 
 #include "common.hpp"
@@ -455,7 +456,7 @@ flash_vt_pipe_kernel(FlashVtParams p) {
 #pragma unroll
     for (int ds = 0; ds < DK; ++ds)  // a half step past the head size re-reads the first dims, times 0
       v[ds] = *reinterpret_cast<const f16x8*>(2 * ds + 1 < DG || g == 0 ? qp + ds * 16 : qp - g * 8);
-    const float cq = qin ? (QS ? p.c : (p.c < 0.0f ? -1.0f : 1.0f)) : 0.0f;
+    const float cq = qin ? (QS ? p.c : (p.c < 0.0f ? -1.0f : p.c == 0.0f ? 0.0f : 1.0f)) : 0.0f;
 #pragma unroll
     for (int ds = 0; ds < DK; ++ds) {
       const float cd = 2 * ds + 1 < DG || g == 0 ? cq : 0.0f;
@@ -464,7 +465,9 @@ flash_vt_pipe_kernel(FlashVtParams p) {
       qf[ds] = v[ds];
     }
   }
-  const float cs = QS ? 1.0f : fabsf(p.c);  // log2 units per score
+  // log2 units per score; never 0, which would turn a masked key's -inf into
+  // NaN (a scale of 0 gives scores of 0 through the sign above)
+  const float cs = QS ? 1.0f : fabsf(p.c) < FLT_MIN ? FLT_MIN : fabsf(p.c);
 
   // Running state, in log2 units: the scores of a tile arrive as s - m with m
   // the lane's current base (negm = -m broadcast is every score chain's

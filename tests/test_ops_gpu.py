@@ -401,6 +401,20 @@ def test_attention_flash_head_dims(gpu, B, H, Sq, Sk, Dh, mul):
     assert float((out.float().cpu() - ref).norm() / ref.norm()) <= 1e-3
 
 
+@pytest.mark.parametrize("Dh", [40, 64, 80])
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-40])
+def test_attention_scale_zero(gpu, scale, Dh):
+    """A scale of (nearly) 0 weighs every key alike and no masked one: the mean of V."""
+    B, H, Sq, Sk = 1, 2, 70, 45
+    announce(f"launch_attention scale {scale} Dh={Dh}")
+    q, k, v = randn((B, H, Sq, Dh), 116), randn((B, H, Sk, Dh), 117), randn((B, H, Sk, Dh), 118)
+    out = torch.empty(B, H, Sq, Dh, dtype=torch.float16, device=gpu)
+    ops.launch_attention(to_gpu(q), to_gpu(k), to_gpu(v), out, B, H, Sq, Sk, Dh, scale)
+    ref = v.double().mean(2, keepdim=True).expand(B, H, Sq, Dh)
+    # one fp16 rounding of O (and, on the general path, one of P)
+    assert float((out.double().cpu() - ref).norm() / ref.norm()) <= 5e-4
+
+
 def test_attention_reference_api_unaligned(gpu):
     """Q / K / V / O that start 2 bytes into their allocation take the general path."""
     B, H, Sq, Sk, Dh = 1, 2, 70, 45, 64
