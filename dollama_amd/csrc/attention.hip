@@ -513,14 +513,19 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   // fp16 values sum to at most 2.1e6).  The first tile (base 0) also moves it
   // down when its row sum is below 2^-8, so the row's largest p is a normal
   // fp16 number and a row whose scores all lie far below 0 cannot underflow
-  // every p.  The rare branch takes the tile's max, re-bases the running
-  // state, this tile and the already issued next tile, and redoes the
-  // exponentials.
+  // every p.  The branch takes the tile's max, re-bases the running state,
+  // this tile and the already issued next tile, and redoes the exponentials.
+  // Head sizes other than 64 always take the max of the first tile (the first
+  // with a score above -inf) as the base:
+  // with base 0, a row whose scores lie around -17 (log2 units) would keep its
+  // P among fp16's subnormals (error 1.7e-3 instead of 3e-4), and the path
+  // they replace held it normalised.
   auto softmax = [&](f32x16 (&sv)[2], f16x8 (&pf)[4], f32x16* sn, bool first) {
     exp_block(sv[0], pf[0], pf[1]);
     exp_block(sv[1], pf[2], pf[3]);
     float lsum = row_sum(pf);
-    const bool low = first && fa_sum_halves(lsum) < (1.0f / 256.0f);
+    const bool fresh = QS ? first : fa_sum_halves(l_run) == 0.0f;
+    const bool low = fresh && (!QS || fa_sum_halves(lsum) < (1.0f / 256.0f));
     if (__builtin_amdgcn_ballot_w64(!(lsum <= 3.0e6f) || low) != 0) {
       asm volatile("" ::: "memory");  // a real branch: never evaluated speculatively
       float mt = sv[0][0];
@@ -529,9 +534,9 @@ flash_vt_pipe_kernel(FlashVtParams p) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) mt = fmaxf(mt, sv[kb][e]);
       mt = fa_max_halves(mt);
-      const float d = first ? mt : fmaxf(mt, 0.0f);
+      const float d = fresh ? (!QS && mt == -INFINITY ? 0.0f : mt) : fmaxf(mt, 0.0f);
       // (the first tile's state is zero; its d may be so low that 2^-d is inf)
-      const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(QS ? -d : -d * cs);
+      const float alpha = fresh ? 1.0f : __builtin_amdgcn_exp2f(QS ? -d : -d * cs);
       l_run *= alpha;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -629,7 +634,8 @@ flash_vt_pipe_kernel(FlashVtParams p) {
   // loop-carried copy of the next tile's 32 scores is needed
   f32x16 sa[2], sb[2];
   // the base starts at 0: tile 0's softmax moves it to that tile's max when
-  // a p overflows or the row's sum is below 2^-8
+  // a p overflows or the row's sum is below 2^-8 (always, for head sizes
+  // other than 64)
 #pragma unroll
   for (int e = 0; e < 16; ++e) negm[e] = 0.0f;
   scores(smem, sa, negm);

@@ -415,6 +415,27 @@ def test_attention_scale_zero(gpu, scale, Dh):
     assert float((out.double().cpu() - ref).norm() / ref.norm()) <= 5e-4
 
 
+@pytest.mark.parametrize("first", [2.5, -2.5, -math.inf])
+@pytest.mark.parametrize("Dh", [40, 80])
+def test_attention_flash_low_rows(gpu, Dh, first):
+    """Head sizes 40 and 80, rows whose scores lie around -12: P stays a normal fp16 number whether
+    the first 64 keys score higher or lower than the rest, or not at all."""
+    B, H, Sq, Sk = 1, 2, 70, 4096
+    announce(f"launch_attention flash low rows Dh={Dh} first keys {first:+}")
+    q = torch.zeros(B, H, Sq, Dh)
+    q[..., 0] = 1.0
+    k, v = randn((B, H, Sk, Dh), 119), randn((B, H, Sk, Dh), 121)
+    k[..., 0] = randn((B, H, Sk), 120, std=0.1, mean=-12.0)
+    k[:, :, :64, 0] += first
+    k = k.half().float()
+    out = torch.empty(B, H, Sq, Dh, dtype=torch.float16, device=gpu)
+    ops.launch_attention(to_gpu(q), to_gpu(k), to_gpu(v), out, B, H, Sq, Sk, Dh, 1.0)
+    s = (q.double() @ k.double().nan_to_num(neginf=-1e5).transpose(-1, -2))
+    ref = torch.softmax(s, -1) @ v.double()
+    # P and O are rounded to fp16, each by at most 2^-11 / sqrt(3) in the mean: 4e-4 together
+    assert float((out.double().cpu() - ref).norm() / ref.norm()) <= 5e-4
+
+
 def test_attention_reference_api_unaligned(gpu):
     """Q / K / V / O that start 2 bytes into their allocation take the general path."""
     B, H, Sq, Sk, Dh = 1, 2, 70, 45, 64
