@@ -2340,11 +2340,15 @@ __global__ void pad_k_kernel(const f16* __restrict__ in, int ld_in, f16* __restr
 
 // The 64 x 64 transposes of both directions (transpose_tile64); image n at
 // n * rows * ld_src and n * cols * ld_out.
+// PIX_ROWS: the pixels are the rows.  They lie on the grid's x, whose limit no
+// image reaches (y ends at 65535 blocks, 2048 x 2048 pixels).
+template <bool PIX_ROWS>
 __global__ void __launch_bounds__(256)
 transpose64_kernel(const f16* __restrict__ in, f16* __restrict__ out, int rows, int cols, int ld_src, int ld_out) {
   __shared__ uint32_t tile[64 * 33];
   transpose_tile64(in + (size_t)blockIdx.z * rows * ld_src, rows, cols, ld_src,
-                   out + (size_t)blockIdx.z * cols * ld_out, ld_out, blockIdx.y * 64, blockIdx.x * 64, tile);
+                   out + (size_t)blockIdx.z * cols * ld_out, ld_out, (PIX_ROWS ? blockIdx.x : blockIdx.y) * 64,
+                   (PIX_ROWS ? blockIdx.y : blockIdx.x) * 64, tile);
 }
 
 // Rows and columns in whole 16-byte vectors take the 64 x 64 tiles, others
@@ -2352,8 +2356,8 @@ transpose64_kernel(const f16* __restrict__ in, f16* __restrict__ out, int rows, 
 // moved: 14.6 -> 9.2 us).
 int nchw_to_nhwc(const void* in, void* out, int N, int C, int HW, int C_pad, hipStream_t s) {
   if (HW % 8 == 0 && C_pad % 8 == 0 && dlm_aligned16(in) && dlm_aligned16(out)) {
-    DLM_LAUNCH("transpose64_kernel", transpose64_kernel, dim3((HW + 63) / 64, (C_pad + 63) / 64, N), dim3(256), 0, s,
-               (const f16*)in, (f16*)out, C, HW, HW, C_pad);
+    DLM_LAUNCH("transpose64_kernel<false>", transpose64_kernel<false>, dim3((HW + 63) / 64, (C_pad + 63) / 64, N),
+               dim3(256), 0, s, (const f16*)in, (f16*)out, C, HW, HW, C_pad);
     DLM_LAUNCH_CHECK();
     return DLM_OK;
   }
@@ -2366,8 +2370,8 @@ int nchw_to_nhwc(const void* in, void* out, int N, int C, int HW, int C_pad, hip
 
 int nhwc_to_nchw(const void* in, void* out, int N, int C, int HW, int C_pad, hipStream_t s) {
   if (HW % 8 == 0 && C % 8 == 0 && C_pad % 8 == 0 && dlm_aligned16(in) && dlm_aligned16(out)) {
-    DLM_LAUNCH("transpose64_kernel", transpose64_kernel, dim3((C + 63) / 64, (HW + 63) / 64, N), dim3(256), 0, s,
-               (const f16*)in, (f16*)out, HW, C, C_pad, HW);
+    DLM_LAUNCH("transpose64_kernel<true>", transpose64_kernel<true>, dim3((HW + 63) / 64, (C + 63) / 64, N), dim3(256),
+               0, s, (const f16*)in, (f16*)out, HW, C, C_pad, HW);
     DLM_LAUNCH_CHECK();
     return DLM_OK;
   }

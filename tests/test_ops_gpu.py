@@ -230,9 +230,10 @@ def test_linear_vt_tiles(gpu, B, S, N, col0, K, ld):
 
 
 @pytest.mark.parametrize("N,C,H,W,cp", [(1, 4, 8, 9, 64), (2, 320, 5, 8, 320), (1, 65, 8, 8, 72), (2, 8, 1, 8, 8),
-                                        (1, 72, 13, 16, 72), (1, 64, 7, 9, 64)])
+                                        (1, 72, 13, 16, 72), (1, 64, 7, 9, 64), (1, 8, 2056, 2056, 8)])
 def test_layout_transposes(gpu, N, C, H, W, cp):
-    """NCHW <-> channels-last: partial tiles, channel padding, and rows that are no whole vectors."""
+    """NCHW <-> channels-last: partial tiles, channel padding, rows that are no whole vectors, and
+    more pixels than the grid's y dimension has room for (65535 blocks of 64)."""
     announce(f"transposes {N}x{C}x{H}x{W} pad {cp}")
     x = to_gpu(randn((N, C, H, W), 129))
     y = ops.nchw_to_nhwc(x, cp)
