@@ -1036,41 +1036,65 @@ __device__ __forceinline__ void vt_tile_store(const f16 DLM_LDS* st, int m0, int
 }
 
 // The same for any token count (77 text tokens) where vt_ld is a multiple of
-// 4: a lane takes four consecutive positions of one sample's V^T row, padding
-// included, and gathers their rows; four that are all this tile's go out as one
-// 8-byte store, the first and last of a tile that splits them one by one.
-// Padding belongs to the tile that holds the sample's last token.  K/V
-// projection of 2 x 77 tokens: 154x2560x2048 20.9 -> 18.9 us, 77x2560x2048
-// 19.5 -> 13.6 us against the per-block form (154x166400x2048 242 -> 220 us
-// against a token per lane).
+// 4.  The tile's rows fall into groups of four positions of a sample's V^T row;
+// the first and last group of a sample in the tile may hold fewer of its rows.
+// A lane finds its group once and walks the columns with it: whole groups go
+// out as 8-byte stores, others position by position, and the lane with a
+// sample's last token clears the row's padding.
+// 154x2560x2048 21.2 -> 16.1 us and 154x166400x2048 207 -> 199 us against the
+// per-block form (19.4 and 215 us where a lane walked every group of the
+// samples it touched, which took 134 us instead of 36 for the LayerNorm-folded
+// QKV of 2 x 999 tokens).
 template <int BM, int BN, int TS, int NT>
 __device__ __forceinline__ void vt_tile_store_any(const f16 DLM_LDS* st, int m0, int n0, const EpiArgs& ep, int tid) {
-  const int tokens = ep.vt_tokens, end = min(m0 + BM, ep.M);
-  const int s0 = m0 / tokens, ns = (end - 1) / tokens - s0 + 1;
-  const int gps = ep.vt_ld >> 2, per = gps * ns;
+  static_assert(BM <= NT, "a lane for every group: each holds at least one row of the tile");
+  const int tokens = ep.vt_tokens, rows = min(BM, ep.M - m0);
+  const int s0 = m0 / tokens, t0 = m0 - s0 * tokens;
+  const int g0 = t0 >> 2, n0g = ((min(tokens, t0 + rows) + 3) >> 2) - g0;  // groups of the first sample
+  const int gps = (tokens + 3) >> 2;                                       // of a whole sample
+  const int more = max(0, rows - (tokens - t0)), whole = more / tokens;    // rows of later samples
+  const int groups = n0g + whole * gps + ((more - whole * tokens + 3) >> 2);
+  const int cs = NT / groups, c0 = tid / groups;
+  if (c0 >= cs) return;
+  int g = tid - c0 * groups, smp = s0, tok = (g0 + g) * 4;
+  if (g >= n0g) {
+    g -= n0g;
+    const int ds = g / gps;
+    smp = s0 + 1 + ds;
+    tok = (g - ds * gps) * 4;
+  }
+  const int r = smp * tokens + tok - m0;         // tile row of the group's first position
+  const bool last = r + tokens - tok <= rows;    // the sample's last token is in the tile
+  const bool tail = last && tok + 4 >= tokens;
   const int vcols = ep.N - ep.vt_col0, cols = min(BN, ep.N - n0);
-  for (int p = tid; p < per * cols; p += NT) {
-    const int c = p / per, q = p - c * per;
-    const int ds = q / gps, tok = (q - ds * gps) * 4;
-    const int base = (s0 + ds) * tokens;  // the sample's first row
-    const bool pad = base + tokens - 1 >= m0 && base + tokens - 1 < end;
-    f16* dst = ep.vt + ((size_t)(s0 + ds) * vcols + (n0 - ep.vt_col0 + c)) * ep.vt_ld + tok;
+  f16* dst = ep.vt + ((size_t)smp * vcols + (n0 - ep.vt_col0 + c0)) * ep.vt_ld + tok;
+  const size_t step = (size_t)cs * ep.vt_ld;
+  const f16 DLM_LDS* src = st + c0 * TS;
+  bool in[4], real[4];
+  int off[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    real[e] = tok + e < tokens;
+    in[e] = real[e] ? r + e >= 0 && r + e < rows : last;
+    off[e] = real[e] && in[e] ? r + e : 0;
+  }
+  const bool all = in[0] && in[1] && in[2] && in[3];
+  for (int c = c0; c < cols; c += cs, dst += step, src += cs * TS) {
     f16x4 v;
-    bool in[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int row = base + tok + e;
-      const bool real = tok + e < tokens;
-      in[e] = real ? row >= m0 && row < end : pad;
-      v[e] = real && in[e] ? st[c * TS + row - m0] : (f16)0.0f;
+      const f16 x = src[off[e]];
+      v[e] = real[e] ? x : (f16)0.0f;
     }
-    if (in[0] && in[1] && in[2] && in[3]) {
+    if (all) {
       *reinterpret_cast<f16x4*>(dst) = v;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (in[e]) dst[e] = v[e];
     }
+    if (tail)
+      for (int q = 4; q < ep.vt_ld - tok; q += 4) *reinterpret_cast<f16x4*>(dst + q) = f16x4{};
   }
 }
 

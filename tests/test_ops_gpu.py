@@ -229,6 +229,30 @@ def test_linear_vt_tiles(gpu, B, S, N, col0, K, ld):
     assert not got[:, :, S:].any()
 
 
+@pytest.mark.parametrize("tile", [8, 11, 14, 24, 35, 44, 45])
+@pytest.mark.parametrize("B,S,N,col0,K,ld", [(2, 999, 400, 160, 64, 1000), (1, 1023, 640, 320, 128, 1024),
+                                             (2, 513, 336, 128, 64, 544), (5, 130, 240, 80, 64, 132),
+                                             (67, 3, 320, 160, 64, 4), (300, 1, 192, 64, 64, 8),
+                                             (2, 77, 640, 160, 192, 80), (2, 260, 400, 240, 64, 260)])
+def test_linear_vt_any_token_count(gpu, B, S, N, col0, K, ld, tile):
+    """Token counts that are no multiple of 4, shorter and longer than a tile, on every tile shape the
+    planner takes: samples that begin and end inside a tile and a group of four, padding after the
+    last token, partial row and column tiles."""
+    from dollama_amd import _lib
+    announce(f"linear_vt forced tile {tile} B={B} S={S} N={N} col0={col0} K={K} ld={ld}")
+    x, w, b = randn((B * S, K), 160), randn((N, K), 161, std=K ** -0.5), randn((N,), 162)
+    try:
+        _lib.call("dlm_gemm_force_tile", tile)
+        y, vt = ops.linear_vt(to_gpu(x), to_gpu(w), col0, S, bias=to_gpu(b), vt_ld=ld)
+    finally:
+        _lib.call("dlm_gemm_force_tile", 0)
+    ref = x @ w.t() + b
+    assert_close(y[:, :col0], ref[:, :col0], "columns before V", rel_tol=5e-4)
+    got = from_gpu(vt).reshape(B, N - col0, ld)
+    assert_close(got[:, :, :S], ref[:, col0:].reshape(B, S, N - col0).transpose(1, 2), "V^T", rel_tol=5e-4)
+    assert not got[:, :, S:].any()
+
+
 @pytest.mark.parametrize("N,C,H,W,cp", [(1, 4, 8, 9, 64), (2, 320, 5, 8, 320), (1, 65, 8, 8, 72), (2, 8, 1, 8, 8),
                                         (1, 72, 13, 16, 72), (1, 64, 7, 9, 64), (1, 8, 2056, 2056, 8)])
 def test_layout_transposes(gpu, N, C, H, W, cp):
