@@ -1961,23 +1961,35 @@ static thread_local int g_forced_tile = 0;
 //   conv 2048x1280x17280 113 -> 99      linear 270x1280x5120 31.5 -> 20.4
 //   linear 2448x640x640 12.1 -> 9.1     linear 988x1280x1280 16.4 -> 12.5
 struct TileCost {
-  int id, bm, bn, slots;
-  float fix, per_slice, per_slice_conv;
+  int id, bm, bn, slots, min_grid;  // min_grid: not for fewer tiles than this
+  float fix, geglu, per_slice, per_slice_conv;  // geglu: added to fix for a GEGLU output
   float split0, split1;  // split0 < 0: never split
 };
-// id as in dlm_gemm_force_tile
+// id as in dlm_gemm_force_tile.  GEGLU: 36 outputs of 60-9500 rows, 10240 x
+// 1280 and 5120 x 640 (6720x5120x640 81 -> 66 us, 1040x5120x640 18.7 -> 16.5
+// against one charge of 2.5 us for the 512-slot tile alone).
 constexpr TileCost kTiles[] = {
-    {45, 256, 160, 256, 9.0f, 1.06f, 1.08f, 15.0f, 1.0f},  {24, 128, 160, 256, 5.0f, 0.72f, 0.76f, 6.0f, 0.5f},
-    {14, 128, 128, 256, 2.5f, 0.60f, 0.60f, 5.0f, 0.7f},   {11, 128, 64, 256, 2.5f, 0.34f, 0.45f, 4.5f, 0.9f},
-    {35, 128, 80, 256, 3.4f, 0.435f, 0.54f, 5.0f, 0.8f},   {29, 128, 128, 512, 3.0f, 1.2f, 1.13f, -1.0f, 0.0f},
-    {19, 256, 128, 256, 7.0f, 0.95f, 0.95f, -1.0f, 0.0f},
+    {45, 256, 160, 256, 0, 9.0f, 0.0f, 1.06f, 1.08f, 15.0f, 1.0f},
+    {24, 128, 160, 256, 0, 5.0f, 0.0f, 0.72f, 0.76f, 6.0f, 0.5f},
+    {14, 128, 128, 256, 0, 2.5f, 1.0f, 0.60f, 0.60f, 5.0f, 0.7f},
+    {11, 128, 64, 256, 0, 2.5f, 0.0f, 0.34f, 0.45f, 4.5f, 0.9f},
+    {35, 128, 80, 256, 0, 3.4f, 0.0f, 0.435f, 0.54f, 5.0f, 0.8f},
+    {29, 128, 128, 512, 256, 3.0f, 1.25f, 1.2f, 1.13f, -1.0f, 0.0f},
+    {19, 256, 128, 256, 0, 7.0f, 0.0f, 0.95f, 0.95f, -1.0f, 0.0f},
 };
-// LayerNorm-folding forms (never split: the row statistics would need a
-// merge of their own)
+// LayerNorm-folding forms (never split: the row statistics would need a merge
+// of their own).  Fits to 108 launches: QKV with V^T, query and GEGLU linears
+// of 60-9500 rows at 640 and 1280 channels, and GEGLU down to one K slice; the
+// choice is the fastest of the six everywhere, within 1%.  A fit to grids of
+// more than 256 tiles alone ran 128x128x4 tiles where 40 is faster, also with
+// one workgroup to a CU (1020x3840x1280 QKV 25.7 -> 22.1 us, start 23.8).
 constexpr TileCost kLnTiles[] = {
-    {41, 256, 160, 256, 9.0f, 1.2f, 1.2f, -1.0f, 0.0f},  {24, 128, 160, 256, 5.0f, 0.95f, 0.95f, -1.0f, 0.0f},
-    {14, 128, 128, 256, 2.5f, 0.75f, 0.75f, -1.0f, 0.0f}, {11, 128, 64, 256, 2.5f, 0.45f, 0.45f, -1.0f, 0.0f},
-    {35, 128, 80, 256, 3.4f, 0.45f, 0.45f, -1.0f, 0.0f},  {40, 128, 128, 512, 3.0f, 1.35f, 1.35f, -1.0f, 0.0f},
+    {41, 256, 160, 256, 0, 8.75f, 0.0f, 1.2f, 1.2f, -1.0f, 0.0f},
+    {24, 128, 160, 256, 0, 4.25f, 0.25f, 0.86f, 0.86f, -1.0f, 0.0f},
+    {14, 128, 128, 256, 0, 2.5f, 1.3f, 0.9f, 0.9f, -1.0f, 0.0f},
+    {11, 128, 64, 256, 0, 2.75f, 0.15f, 0.52f, 0.52f, -1.0f, 0.0f},
+    {35, 128, 80, 256, 0, 2.4f, 0.75f, 0.49f, 0.49f, -1.0f, 0.0f},
+    {40, 128, 128, 512, 0, 2.0f, 2.5f, 1.35f, 1.35f, -1.0f, 0.0f},
 };
 constexpr int kMaxSplits = 12;
 struct GemmPlan {
@@ -1989,11 +2001,10 @@ static GemmPlan plan_gemm(const TileCost (&tiles)[NT], int M, int N, int nk, boo
   float best_t = 3e38f;
   for (const TileCost& t : tiles) {
     const long long grid = ceil_div(M, t.bm) * ceil_div(N, t.bn);
-    // two workgroups to a CU only pay where both have a tile; 256x128 only for
-    // convs of up to four 128x128 tiles per CU (larger grids keep 128x128,
-    // whose fp32 epilogues pass under the other workgroup's main loop: VAE
-    // decode 17.0 against 17.4 ms)
-    if (t.slots == 512 && grid < 256) continue;
+    // 256x128 only for convs of up to four 128x128 tiles per CU (larger grids
+    // keep 128x128, whose fp32 epilogues pass under the other workgroup's main
+    // loop: VAE decode 17.0 against 17.4 ms)
+    if (grid < t.min_grid) continue;
     if (t.id == 19 && (!conv || ceil_div(M, 128) * ceil_div(N, 128) >= 4 * 256)) continue;
     for (int S = 1; S <= max_splits && S <= nk; ++S) {
       if (S > 1 && (t.split0 < 0.0f || (size_t)grid * S * t.bm * t.bn > kSplitWsFloats || grid > kSplitCounters)) break;
@@ -2002,7 +2013,7 @@ static GemmPlan plan_gemm(const TileCost (&tiles)[NT], int M, int N, int nk, boo
       // a last round with one workgroup to a CU instead of two runs faster
       float rounds = (float)ceil_div(grid * S, t.slots);
       if (t.slots == 512 && grid % 512 >= 1 && grid % 512 <= 256) rounds -= 0.4f;
-      const float fix = t.fix + (geglu && t.slots == 512 ? 2.5f : 0.0f);
+      const float fix = t.fix + (geglu ? t.geglu : 0.0f);
       const float us = rounds * (fix + (float)kps * (conv ? t.per_slice_conv : t.per_slice)) +
                        (S > 1 ? t.split0 + (float)S * t.split1 : 0.0f);
       if (us < best_t) {
