@@ -186,10 +186,11 @@ def test_conv_nhwc_concat_shortcut_residual_tbias(gpu):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 320, 640), (63, 1284, 5128), (144, 1280, 5120), (257, 640, 2560),
-                                   (532, 1280, 5120), (1224, 640, 2568)])
+                                   (532, 1280, 5120), (1224, 640, 2568), (1, 216, 8), (512, 1024, 2560),
+                                   (513, 1024, 2624), (257, 1020, 2568), (1280, 640, 2560), (2089, 260, 3528)])
 def test_linear_planned_splits(gpu, M, N, K):
-    """Grids that leave CUs idle take small tiles and split-K: partial tiles, a K tail that ends inside
-    the last split, and the same result on every launch."""
+    """Grids that leave CUs idle take small tiles and split-K, the 64 x 16 tiles or the register-staged
+    kernel: partial tiles, a K tail that ends inside the last split, and the same result on every launch."""
     announce(f"linear planned splits {M}x{N}x{K}")
     x, w, b, r = randn((M, K), 120), randn((N, K), 121, std=K ** -0.5), randn((N,), 122), randn((M, N), 123)
     args = dict(bias=to_gpu(b), residual=to_gpu(r))
@@ -202,7 +203,8 @@ def test_linear_planned_splits(gpu, M, N, K):
 
 @pytest.mark.parametrize("B,H,W,Ci,Co,stride,up", [(1, 1, 1, 640, 1280, 1, False), (1, 12, 20, 1280, 1280, 1, False),
                                                    (2, 15, 17, 640, 320, 2, False), (1, 9, 7, 640, 640, 1, True),
-                                                   (2, 16, 8, 320, 1280, 1, False)])
+                                                   (2, 16, 8, 320, 1280, 1, False), (1, 1, 3, 64, 1552, 1, False),
+                                                   (2, 7, 9, 128, 320, 1, True)])
 def test_conv_planned_splits(gpu, B, H, W, Ci, Co, stride, up):
     """The same for 3x3 convs: one pixel, odd sizes, strides, upsampling."""
     announce(f"conv planned splits {B}x{H}x{W} {Ci}-{Co} s{stride} up{up}")
