@@ -43,7 +43,8 @@ int dlm_gemm_force_tile(int tile_id);
 int dlm_gemm_override_shape(int M, int N, int K, int tile_id, int splits);
 int dlm_gemm_force_split(int splits);
 /* Tuning aid: select alternative tile heuristics (0 = default; bit 0 = plans
- * without split-K). */
+ * without split-K; bit 1 = a stream's split-K workspace cannot be allocated,
+ * as on a full device). */
 int dlm_gemm_set_variant(int variant);
 
 /* Counter calibration: `blocks` workgroups of 4 waves, each wave `iters`

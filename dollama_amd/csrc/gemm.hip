@@ -1756,41 +1756,65 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
 // order and share it; another stream gets its own.  Sized once; a launch
 // that would need more falls back to one split.
 struct SplitWorkspace {
-  float* ws = nullptr;
+  float* ws = nullptr;  // partials, then the arrival counters, in one block
   int* cnt = nullptr;
+  int wait = 0;  // requests to turn away before the allocation is tried again
 };
 constexpr size_t kSplitWsFloats = size_t(24) << 20;  // 96 MiB of fp32 partials
 constexpr int kSplitCounters = 1 << 16;
+// dlm_gemm_set_variant (tuning aids below); bit 1: the workspace's allocation
+// asks for more than any device holds
+static thread_local int g_variant = 0;
 static std::mutex g_split_mu;
 static std::map<std::pair<int, hipStream_t>, SplitWorkspace> g_split_ws;
 
-// A stream under graph capture gets no new workspace (the allocation and its
-// synchronous clear would invalidate the capture): its launches run unsplit
-// until the stream has made one outside capture.
+__global__ void zero_ints_kernel(int* p, int n) { GRID_STRIDE(i, n) p[i] = 0; }
+
+// A stream under graph capture gets no new workspace: its launches run
+// unsplit until the stream has made one outside capture.  Another stream's
+// capture, on this thread or another, is left alone: the allocation runs in
+// the relaxed capture mode, and the counters are cleared by a kernel on `s`,
+// in order before the launch that needs them, so nothing synchronises.  Where
+// the memory is not to be had, launches run unsplit, the failed call's error
+// does not stay behind for them to report, and the next attempt waits for a
+// thousand requests.
 static const SplitWorkspace* split_workspace(hipStream_t s) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return nullptr;
   std::lock_guard<std::mutex> lk(g_split_mu);
   auto it = g_split_ws.find({dev, s});
   if (it != g_split_ws.end() && it->second.ws) return &it->second;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
-  SplitWorkspace& w = g_split_ws[{dev, s}];
-  if (!w.ws) {
-    float* ws = nullptr;
-    int* cnt = nullptr;
-    if (hipMalloc(&ws, kSplitWsFloats * sizeof(float)) != hipSuccess) return nullptr;
-    if (hipMalloc(&cnt, kSplitCounters * sizeof(int)) != hipSuccess ||
-        hipMemset(cnt, 0, kSplitCounters * sizeof(int)) != hipSuccess ||
-        hipDeviceSynchronize() != hipSuccess) {
-      (void)hipFree(ws);
-      if (cnt) (void)hipFree(cnt);
-      return nullptr;
-    }
-    w.ws = ws;
-    w.cnt = cnt;
+  if (it != g_split_ws.end() && it->second.wait > 0) {
+    --it->second.wait;
+    return nullptr;
   }
-  return &w;
+  if (hipPeekAtLastError() != hipSuccess) return nullptr;  // not ours: the launch reports it
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (cap != hipStreamCaptureStatusNone) return nullptr;
+  SplitWorkspace& w = g_split_ws[{dev, s}];
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  float* ws = nullptr;
+  const size_t bytes = kSplitWsFloats * sizeof(float) + kSplitCounters * sizeof(int);
+  const hipError_t e = hipMalloc(&ws, g_variant & 2 ? size_t(1) << 60 : bytes);
+  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (e == hipSuccess) {
+    int* cnt = reinterpret_cast<int*>(ws + kSplitWsFloats);
+    hipLaunchKernelGGL(zero_ints_kernel, dim3(64), dim3(256), 0, s, cnt, kSplitCounters);
+    if (hipPeekAtLastError() == hipSuccess) {
+      w.ws = ws;
+      w.cnt = cnt;
+      return &w;
+    }
+    (void)hipFree(ws);
+  }
+  (void)hipGetLastError();
+  w.wait = 1000;
+  return nullptr;
 }
 
 // Frees the split-K workspace of `s` on every device (after synchronising
@@ -1804,8 +1828,7 @@ int split_workspace_release(hipStream_t s) {
   if (hipStreamSynchronize(s) != hipSuccess) return fail(DLM_ERR_HIP, "split workspace: stream synchronisation failed");
   for (auto it = g_split_ws.begin(); it != g_split_ws.end();) {
     if (it->first.second == s) {
-      if ((it->second.ws && hipFree(it->second.ws) != hipSuccess) ||
-          (it->second.cnt && hipFree(it->second.cnt) != hipSuccess))
+      if (it->second.ws && hipFree(it->second.ws) != hipSuccess)
         return fail(DLM_ERR_HIP, "split workspace: hipFree failed");
       it = g_split_ws.erase(it);
     } else {
@@ -1827,7 +1850,6 @@ size_t split_workspace_bytes() {
 // _override_shape): thread-local, so they steer only launches made by the
 // thread that set them.
 static thread_local int g_forced_split = 0;
-static thread_local int g_variant = 0;  // bits select alternative heuristics
 // Set while an allocation-free entry point runs: split-K stays off, since its
 // workspace is allocated on first use.
 static thread_local bool t_no_split = false;

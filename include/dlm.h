@@ -96,7 +96,9 @@ int dlm_mem_get_info(size_t* free_bytes, size_t* total_bytes);
  * 2 GiB.  dlm_scratch_release synchronises `stream` and frees everything
  * the library holds for it: call it before destroying a stream that ran
  * library entry points (a new stream may reuse the handle).  Graphs captured
- * on that stream must not be replayed afterwards.  No reference counterpart
+ * on that stream must not be replayed afterwards, and graphs captured on one
+ * stream share its split-K workspace: two of them, or one and work that runs
+ * on the stream itself, must not run at the same time.  No reference counterpart
  * (the reference's launch_* wrappers cudaMalloc / cudaFree per call).
  * dlm_scratch_bytes reports the device bytes the library holds for all
  * streams. */

@@ -71,3 +71,67 @@ def test_streams_cycled_through_reference_entries_give_memory_back(gpu):
     _release(streams[0])
     assert _held() <= base
     print(f"[scratch] {per_stream / 2**20:.1f} MiB per stream, all returned", flush=True)
+
+
+def test_split_workspace_that_cannot_be_had(gpu):
+    """A GEMM whose plan splits K runs unsplit when its stream's workspace cannot be allocated: no
+    error of the failed allocation is left for the launch to report, and once the stream's state is
+    released the split form's bits come back."""
+    M, N, K = 144, 1280, 5120
+    print(f"[case] linear {M}x{N}x{K} on a stream without a split-K workspace", flush=True)
+    x, w = to_gpu(randn((M, K), 7)), to_gpu(randn((N, K), 8, std=K ** -0.5))
+    want = ops.linear(x, w)
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()
+    _release(st)
+    try:
+        with torch.cuda.stream(st):
+            _lib.call("dlm_gemm_set_variant", 1)
+            unsplit = ops.linear(x, w)
+            _lib.call("dlm_gemm_set_variant", 2)
+            held = _held()
+            for _ in range(3):
+                assert torch.equal(ops.linear(x, w), unsplit)
+            assert _held() == held
+            st.synchronize()
+            _release(st)
+            _lib.call("dlm_gemm_set_variant", 0)
+            assert torch.equal(ops.linear(x, w), want)
+            assert _held() > held
+            st.synchronize()
+    finally:
+        _lib.call("dlm_gemm_set_variant", 0)
+        _release(st)
+
+
+def test_split_workspace_during_another_streams_capture(gpu):
+    """A stream gets its split-K workspace while another stream is captured, without disturbing the
+    capture; the captured stream itself, which has none, runs unsplit."""
+    M, N, K = 144, 1280, 5120
+    print(f"[case] linear {M}x{N}x{K} while another stream is captured", flush=True)
+    x, w = to_gpu(randn((M, K), 9)), to_gpu(randn((N, K), 10, std=K ** -0.5))
+    want = ops.linear(x, w)
+    try:
+        _lib.call("dlm_gemm_set_variant", 1)
+        unsplit = ops.linear(x, w)
+    finally:
+        _lib.call("dlm_gemm_set_variant", 0)
+    ya, yb = torch.empty_like(want), torch.empty_like(want)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    _release(a)
+    _release(b)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=a):
+        ops.linear(x, w, out=ya)
+        with torch.cuda.stream(b):
+            ops.linear(x, w, out=yb)
+    b.synchronize()
+    assert torch.equal(yb, want)
+    for _ in range(3):
+        ya.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ya, unsplit)
+        assert torch.equal(ops.linear(x, w), want)
+    _release(b)
