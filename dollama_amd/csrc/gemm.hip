@@ -1242,6 +1242,8 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
   static_assert(BM % 8 == 0 && BN % 8 == 0 && WM % 16 == 0 && WN % 16 == 0, "tile shape");
   static_assert(NS >= 2, "at least two slices");
   static_assert(SPS == 1 || SCH == kPlain, "multi-slice stages use the plain loop");
+  static_assert(!LNS || SCH != kPingPong, "no LayerNorm statistics in the ping-pong loop");
+  static_assert(NW % 2 == 0, "RowDma: a lane's chunk is the same in all its DMA instructions");
   __shared__ __attribute__((aligned(1024))) unsigned char smem_generic[NS * STAGE];
   unsigned char DLM_LDS* smem = (unsigned char DLM_LDS*)smem_generic;
 
@@ -1476,7 +1478,6 @@ dma_gemm_kernel(Desc ad, RowDesc bd, EpiArgs ep, int tiles_m, int tiles_n, Split
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x32(fb[j], fa[i], acc[i][j]);
-        ln_acc(fa);
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
@@ -1879,7 +1880,7 @@ constexpr bool ln_tile() {
          (BM == 128 && BN == 128 && WM == 64 && WN == 32 && SPS == 1) ||
          (BM == 128 && BN == 64 && WM == 64 && WN == 32 && NS == 4 && SPS == 1) ||
          (BM == 128 && BN == 128 && WM == 32 && WN == 64 && NS == 2 && SPS == 1) ||
-         (BM == 256 && BN == 160 && WM == 64 && WN == 80 && NS == 3 && SPS == 1) ||
+         (BM == 256 && BN == 160 && WM == 64 && WN == 80 && NS == 3 && SCH != kPingPong && SPS == 1) ||
          (BM == 256 && BN == 160 && WM == 32 && WN == 160 && NS == 3 && SPS == 1) ||
          (BM == 128 && BN == 160 && WM == 32 && WN == 80 && SPS == 1);
 }
@@ -2121,7 +2122,6 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
         case 35: return launch_dma<128, 80, 16, 80, 3, kPlain, 2>(ad, bd, ep, M, N, s);
         case 40: return launch_dma<128, 128, 32, 64, 2, kPrefetch>(ad, bd, ep, M, N, s);
         case 41: return launch_dma<256, 160, 32, 160, 3, kPrefetch>(ad, bd, ep, M, N, s);
-        case 45: return launch_dma<256, 160, 64, 80, 3, kPingPong>(ad, bd, ep, M, N, s);
         case 0: break;
         default: return fail(DLM_ERR_UNSUPPORTED, "forced tile has no LayerNorm-folding kernel");
       }
