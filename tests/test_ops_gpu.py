@@ -55,11 +55,11 @@ def test_linear_geglu(gpu, M, d, K):
     assert_close(y, R.geglu(R.linear(x, w, b)), f"geglu {M}x{d}x{K}")
 
 
-@pytest.mark.parametrize("tile", list(range(8, 45)))
+@pytest.mark.parametrize("tile", list(range(8, 46)))
 def test_dma_tile_configs(gpu, tile):
-    """Every LDS-DMA tile configuration (dlm_gemm_force_tile 8-44, the
+    """Every LDS-DMA tile configuration (dlm_gemm_force_tile 8-45, the
     fragment-prefetch forms 27-34, two-slice stages 35-39, the 16-column
-    tiles 42-43 and the 192-row tile 44 included),
+    tiles 42-43, the 192-row tile 44 and the ping-pong tile 45 included),
     whole and split-K, on ragged shapes with an odd slice count and a K tail:
     bias + SiLU + residual, GEGLU, and a 3x3 conv with residual."""
     from dollama_amd import _lib
@@ -84,6 +84,32 @@ def test_dma_tile_configs(gpu, tile):
         wp, bp = ops.pack_geglu(to_gpu(wg), to_gpu(bg))
         yg = ops.linear(to_gpu(x), wp, bias=bp, act=ops.ACT_GEGLU)
         assert_close(yg, R.geglu(R.linear(x, wg, bg)), f"tile {tile} geglu")
+    finally:
+        _lib.call("dlm_gemm_force_tile", 0)
+        _lib.call("dlm_gemm_force_split", 0)
+
+
+@pytest.mark.parametrize("K", [64, 200, 648, 1280])
+@pytest.mark.parametrize("tile", [11, 14, 24, 35, 45])
+def test_planned_tiles_short_splits(gpu, tile, K):
+    """The tiles whose plans split K, with ranges down to one and two slices (fewer than the ring
+    holds), a K tail, and partial row and column tiles: linear and 3x3 conv (nine slices)."""
+    from dollama_amd import _lib
+    M, N = 300, 340
+    x, w, b = randn((M, K), 163), randn((N, K), 164, std=K ** -0.5), randn((N,), 165)
+    xc, wc = randn((1, 64, 19, 17), 166), randn((340, 64, 3, 3), 167, std=1 / 24)
+    ref, refc = x @ w.t() + b, torch.nn.functional.conv2d(xc, wc, padding=1)
+    try:
+        _lib.call("dlm_gemm_force_tile", tile)
+        for splits in (1, 2, 5, 6, 11):
+            announce(f"forced tile {tile} K={K} splits {splits}")
+            _lib.call("dlm_gemm_force_split", splits)
+            y = ops.linear(to_gpu(x), to_gpu(w), bias=to_gpu(b))
+            # fp32 sums in another order and one fp16 rounding (2^-11 of the value)
+            assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
+            if K == 64:
+                yc = ops.conv2d_nhwc(ops.nchw_to_nhwc(to_gpu(xc)), ops.pack_conv_weight(to_gpu(wc)), KH=3, KW=3, pad=1)
+                assert float((from_gpu(ops.nhwc_to_nchw(yc)) - refc).norm() / refc.norm()) <= 5e-4
     finally:
         _lib.call("dlm_gemm_force_tile", 0)
         _lib.call("dlm_gemm_force_split", 0)
@@ -625,6 +651,36 @@ def test_linear_layernorm_folded(gpu, M, N, K, act, vt):
     else:
         y = ops.linear_ln(to_gpu(x), wf, c1, c2, 1e-5, act=act)
         assert_close(y, ref, "linear_ln")
+
+
+@pytest.mark.parametrize("tile", [11, 14, 24, 28, 29, 31, 35, 40, 41])
+@pytest.mark.parametrize("B,S,K", [(2, 77, 64), (1, 259, 192), (3, 100, 320), (2, 260, 64)])
+def test_linear_layernorm_folded_tiles(gpu, B, S, K, tile):
+    """Every LayerNorm-folding tile: plain with residual, GEGLU and transposed V, on one to five K
+    slices, partial row and column tiles, and token counts that are and are not multiples of 4."""
+    from dollama_amd import _lib
+    announce(f"linear_ln forced tile {tile} B={B} S={S} K={K}")
+    M, C, ld = B * S, 112, (S + 7) & ~7
+    x = randn((M, K), 168, std=2.0, mean=0.5)
+    g, b = randn((K,), 169, std=0.3, mean=1.0), randn((K,), 170, std=0.3)
+    w, bias, r = randn((3 * C, K), 171, std=K ** -0.5), randn((3 * C,), 172, std=0.1), randn((M, 3 * C), 173)
+    ref = R.linear(R.layer_norm(x, g, b, 1e-5), w, bias)
+    wf, c1, c2 = ops.ln_fold(to_gpu(w), to_gpu(g), to_gpu(b), to_gpu(bias))
+    wp, bp = ops.pack_geglu(to_gpu(w), to_gpu(bias))
+    gf, g1, g2 = ops.ln_fold(wp, to_gpu(g), to_gpu(b), bp)
+    try:
+        _lib.call("dlm_gemm_force_tile", tile)
+        y = ops.linear_ln(to_gpu(x), wf, c1, c2, 1e-5, residual=to_gpu(r))
+        yg = ops.linear_ln(to_gpu(x), gf, g1, g2, 1e-5, act=ops.ACT_GEGLU)
+        yq, vt = ops.linear_vt_ln(to_gpu(x), wf, c1, c2, 1e-5, 2 * C, S, vt_ld=ld)
+    finally:
+        _lib.call("dlm_gemm_force_tile", 0)
+    assert_close(y, ref + r, "linear_ln + residual")
+    assert_close(yg, R.geglu(ref), "linear_ln geglu")
+    assert_close(yq, ref[:, :2 * C], "linear_vt_ln y")
+    got = from_gpu(vt).reshape(B, C, ld)
+    assert_close(got[:, :, :S], ref[:, 2 * C:].reshape(B, S, C).transpose(1, 2), "linear_vt_ln vt")
+    assert not got[:, :, S:].any()
 
 
 def test_linear_layernorm_folded_large_offset(gpu):
