@@ -241,19 +241,25 @@ __global__ void gn_finalize_kernel(const float2* __restrict__ partial, int HW, i
   }
 }
 
+// First thread of a short last chunk, after `full` whole ones of S threads
+__host__ __device__ __forceinline__ int gn_chan_tail(int full, int S) { return (full * S + 63) & ~63; }
+
 // Per-channel chunk statistics of fp16 [N, HW, C] (+ concatenated second
 // source): one thread per (chunk, 4-channel vector), the chunk's rows in
 // ascending order.  A whole chunk's 64 rows are requested before the first is
 // used (128 VGPRs): one memory round trip.  Eight rows of 8 channels in
 // flight made eight of them on half the waves, which bounded the kernel at any
-// size (2x64x64x960, 15.7 MB: 10.1 -> 6.9 us).
+// size (2x64x64x960, 15.7 MB: 10.1 -> 6.3 us).
 __global__ void __launch_bounds__(256)
 gn_chan_stats_kernel(const f16* __restrict__ a, int Ca, int lda, const f16* __restrict__ b, int ldb,
                      int HW, int C, int S, int chunks, float2* __restrict__ stats) {
   const int n = blockIdx.y;
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = idx / S, s = idx - k * S;
-  if (k >= chunks) return;
+  // whole chunks first; a short last one starts at a wave of its own, since
+  // it takes the other path below
+  const int full = HW / kGnChunk, tail = gn_chan_tail(full, S);
+  const int k = idx < full * S ? idx / S : full, s = idx < full * S ? idx - k * S : idx - tail;
+  if (k >= chunks || s < 0 || s >= S) return;
   const int c = s * 4;
   const f16* src;
   int ld;
@@ -269,28 +275,46 @@ gn_chan_stats_kernel(const f16* __restrict__ a, int Ca, int lda, const f16* __re
   float shift[4], s1[4], s2[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) s1[i] = s2[i] = 0.0f;
-  // the last chunk of a sample may be short: rows past it re-read its last row
-  // and count as the shift, whose d = 0 leaves both sums as they are
-  auto run = [&](auto whole) {
+  if (cnt == kGnChunk) {
     f16x4 v[kGnChunk];
 #pragma unroll
-    for (int u = 0; u < kGnChunk; ++u)
-      v[u] = *reinterpret_cast<const f16x4*>(src + (size_t)(decltype(whole)::value ? u : min(u, cnt - 1)) * ld);
+    for (int u = 0; u < kGnChunk; ++u) v[u] = *reinterpret_cast<const f16x4*>(src + (size_t)u * ld);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) shift[i] = (float)v[0][i];
 #pragma unroll
     for (int u = 0; u < kGnChunk; ++u)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float x = (float)v[u][i];
-        gn_stat_add(decltype(whole)::value || u < cnt ? x : shift[i], shift[i], s1[i], s2[i]);
-      }
-  };
-  if (cnt == kGnChunk) {
-    run(std::true_type{});
+      for (int i = 0; i < 4; ++i) gn_stat_add((float)v[u][i], shift[i], s1[i], s2[i]);
   } else {
-    run(std::false_type{});
+    // The last chunk of a sample may be short: 8 or 16 rows at a time, of
+    // which those past the end re-read the last row and count as the shift,
+    // whose d = 0 leaves both sums as they are.  (All 64 at once cost an image
+    // of 2x2 pixels 6.3 us against 2.9; 32 at a time were slower than 16 for
+    // 35-41 rows.)
+    auto rows = [&](auto count) {
+      constexpr int R = decltype(count)::value;
+#pragma unroll 1
+      for (int r = 0; r < cnt; r += R) {
+        f16x4 v[R];
+#pragma unroll
+        for (int u = 0; u < R; ++u) v[u] = *reinterpret_cast<const f16x4*>(src + (size_t)min(r + u, cnt - 1) * ld);
+        __builtin_amdgcn_sched_barrier(0);
+        if (r == 0) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) shift[i] = (float)v[0][i];
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) gn_stat_add(r + u < cnt ? (float)v[u][i] : shift[i], shift[i], s1[i], s2[i]);
+      }
+    };
+    if (cnt <= 8) {
+      rows(std::integral_constant<int, 8>{});
+    } else {
+      rows(std::integral_constant<int, 16>{});
+    }
   }
   float4* dst = reinterpret_cast<float4*>(stats + ((size_t)n * chunks + k) * C + c);
 #pragma unroll
@@ -470,7 +494,8 @@ __global__ void gn_apply_kernel(const T* __restrict__ a, int Ca, int lda,
 static int gn_chan_stats_launch(const f16* a, int C_a, int ld_a, const f16* b, int ld_b, int N,
                                 int HW, int C, float2* stats, hipStream_t s) {
   const int S = C / 4, chunks = gn_chan_chunks(HW);
-  DLM_LAUNCH("gn_chan_stats_kernel", gn_chan_stats_kernel, dim3((chunks * S + 255) / 256, N), dim3(256), 0, s, a,
+  const int full = HW / kGnChunk, threads = full < chunks ? gn_chan_tail(full, S) + S : full * S;
+  DLM_LAUNCH("gn_chan_stats_kernel", gn_chan_stats_kernel, dim3((threads + 255) / 256, N), dim3(256), 0, s, a,
              C_a, ld_a, b, ld_b, HW, C, S, chunks, stats);
   DLM_LAUNCH_CHECK();
   return DLM_OK;

@@ -105,12 +105,17 @@ def test_linear_gn_stats_equal_stats_pass(gpu, tile):
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,C,H,W,mean,std", [(2, 320, 128, 128, 0.0, 1.0), (2, 640, 64, 64, 40.0, 0.5),
                                               (1, 1280, 32, 32, -3.0, 2.0), (3, 64, 9, 7, 0.5, 1.5),
-                                              (1, 1024, 128, 128, 0.0, 1.0), (1, 1280, 127, 121, 1.0, 1.0)])
+                                              (1, 1024, 128, 128, 0.0, 1.0), (1, 1280, 127, 121, 1.0, 1.0),
+                                              (2, 64, 1, 4, 40.0, 0.5), (1, 320, 3, 3, 0.0, 1.0),
+                                              (3, 320, 4, 4, 1.0, 1.0), (2, 96, 1, 17, 0.0, 1.0),
+                                              (2, 1280, 5, 13, 40.0, 0.5), (2, 96, 3, 35, 0.0, 1.0)])
 def test_group_norm_chunk_statistics_vs_oracle(gpu, N, C, H, W, mean, std):
     """GroupNorm(+SiLU) over the chunk statistics (the path of every fp16
     GroupNorm of up to 16384 pixels) against the float64 oracle on the same
     fp16 values, at the UNet's three level shapes, a mean 80x the standard
-    deviation, a pixel count that leaves a partial last chunk, groups of
+    deviation, pixel counts that leave a partial last chunk (of 1 to 63 rows,
+    the only one or after whole ones, at channel counts that do and do not
+    fill waves), groups of
     exactly as many entries as the merge holds in registers (256 chunks x 32
     channels) and of more (241 chunks x 40 channels); the prestats form from
     the statistics pass gives the same bits."""
