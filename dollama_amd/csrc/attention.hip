@@ -964,7 +964,7 @@ static int attention_reference_layout(const f16* q, const f16* k, const f16* v, 
   const int K8 = (Sk + 7) & ~7;
   int st = DLM_OK;
   // Head sizes of the SD and SDXL UNets: the flash kernel (2 x 10 heads x 2259
-  // tokens x 80: 77 us against 969 us for a GEMM, softmax and GEMM per head).
+  // tokens x 80: 78 us against 969 us for a GEMM, softmax and GEMM per head).
   // Any other size, and operands that are not aligned, take those per head.
   const bool vt_fits = (unsigned long long)BH * Dh * K8 * 2 < (1ull << 31);
   if ((Dh == 64 || ((Dh == 40 || Dh == 80) && vt_fits)) && dlm_aligned16(q) && dlm_aligned16(k) &&

@@ -25,7 +25,7 @@
 //     the current k-step's MFMAs.  Optional split-K with a last-arriver
 //     reduction in split order, and an XCD-aware tile order.
 //   - mfma_gemm_kernel (small channel counts, kernels over 14 taps, unaligned
-//     operands): 4 waves of 32x32x16 MFMA blocks with VGPR-staged,
+//     operands, linears of about one 64x64 tile per CU): 4 waves of 32x32x16 MFMA blocks with VGPR-staged,
 //     double-buffered LDS slices (row stride 72 halfs).
 // The A operand is produced by a loader: plain rows for linears, or the
 // implicit im2col gather (zero padding, channel concatenation of two
@@ -1217,7 +1217,13 @@ __device__ __forceinline__ void split_coords(int bid, int tiles_m, int tiles_n, 
 // either half reads it.  256x160 tile, 64x80 waves: 1690 cycles a slice, of
 // which the MFMAs are 1280 (1290 with the DMA or the reads taken out), at the
 // 1.6 GHz that the power limit leaves; the plain loop needs 10% more.
-// 2048x10240x1280 GEGLU 71 -> 65 us, 4096x2560x5120 112 -> 100 us.  Smaller
+// 2048x10240x1280 GEGLU 71 -> 65 us, 4096x2560x5120 112 -> 100 us; weights and
+// inputs that no cache holds 68.6 -> 62.2 us.  Inside a whole UNet step the 60
+// GEGLU launches gain 0.35 ms over the prefetch schedule and 0.12 ms over the
+// plain one, but the power they take slows the launches around them by more:
+// with FF1 on the prefetch schedule the step measured 0.30-0.32 ms faster on
+// two boxes and 0.03 slower on a third, on the plain one 0.10-0.21 ms faster
+// on four.  Launches that run alone keep the ping-pong.  Smaller
 // tiles, whose read phases are longer than their MFMA phases, measured slower
 // with it (128x128: 29 -> 34 us at 2048x3840x1280).
 // SPS > 1: a ring stage holds SPS consecutive K slices published by one
