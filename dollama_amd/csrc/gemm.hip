@@ -1991,20 +1991,22 @@ static thread_local int g_forced_tile = 0;
 //   linear 2448x640x640 12.1 -> 9.1     linear 988x1280x1280 16.4 -> 12.5
 struct TileCost {
   int id, bm, bn, slots, min_grid;  // min_grid: not for fewer tiles than this
-  float fix, geglu, per_slice, per_slice_conv;  // geglu: added to fix for a GEGLU output
+  float fix, geglu, conv, per_slice, per_slice_conv;  // geglu, conv: added to fix for these
   float split0, split1;  // split0 < 0: never split
 };
 // id as in dlm_gemm_force_tile.  GEGLU: 36 outputs of 60-9500 rows, 10240 x
 // 1280 and 5120 x 640 (6720x5120x640 81 -> 66 us, 1040x5120x640 18.7 -> 16.5
-// against one charge of 2.5 us for the 512-slot tile alone).
+// against one charge of 2.5 us for the 512-slot tile alone).  Conv: what the
+// loader's set-up adds on the two 128x128 forms, from 200 convs of 5-45 slices
+// (1x1 8000x1280x320 21.6 -> 18.9 us, 8192x640x320 14.8 -> 12.4).
 constexpr TileCost kTiles[] = {
-    {45, 256, 160, 256, 0, 9.0f, 0.0f, 1.06f, 1.08f, 15.0f, 1.0f},
-    {24, 128, 160, 256, 0, 5.0f, 0.0f, 0.72f, 0.76f, 6.0f, 0.5f},
-    {14, 128, 128, 256, 0, 2.5f, 1.0f, 0.60f, 0.60f, 5.0f, 0.7f},
-    {11, 128, 64, 256, 0, 2.5f, 0.0f, 0.34f, 0.45f, 4.5f, 0.9f},
-    {35, 128, 80, 256, 0, 3.4f, 0.0f, 0.435f, 0.54f, 5.0f, 0.8f},
-    {29, 128, 128, 512, 256, 3.0f, 1.25f, 1.2f, 1.13f, -1.0f, 0.0f},
-    {19, 256, 128, 256, 0, 7.0f, 0.0f, 0.95f, 0.95f, -1.0f, 0.0f},
+    {45, 256, 160, 256, 0, 9.0f, 0.0f, 0.0f, 1.06f, 1.08f, 15.0f, 1.0f},
+    {24, 128, 160, 256, 0, 5.0f, 0.0f, 0.0f, 0.72f, 0.76f, 6.0f, 0.5f},
+    {14, 128, 128, 256, 0, 2.5f, 1.0f, 1.0f, 0.60f, 0.60f, 5.0f, 0.7f},
+    {11, 128, 64, 256, 0, 2.5f, 0.0f, 0.0f, 0.34f, 0.45f, 4.5f, 0.9f},
+    {35, 128, 80, 256, 0, 3.4f, 0.0f, 0.0f, 0.435f, 0.54f, 5.0f, 0.8f},
+    {29, 128, 128, 512, 256, 3.0f, 1.25f, 1.75f, 1.2f, 1.13f, -1.0f, 0.0f},
+    {19, 256, 128, 256, 0, 7.0f, 0.0f, 0.0f, 0.95f, 0.95f, -1.0f, 0.0f},
 };
 // LayerNorm-folding forms (never split: the row statistics would need a merge
 // of their own).  Fits to 108 launches: QKV with V^T, query and GEGLU linears
@@ -2013,12 +2015,12 @@ constexpr TileCost kTiles[] = {
 // more than 256 tiles alone ran 128x128x4 tiles where 40 is faster, also with
 // one workgroup to a CU (1020x3840x1280 QKV 25.7 -> 22.1 us, start 23.8).
 constexpr TileCost kLnTiles[] = {
-    {41, 256, 160, 256, 0, 8.75f, 0.0f, 1.2f, 1.2f, -1.0f, 0.0f},
-    {24, 128, 160, 256, 0, 4.25f, 0.25f, 0.86f, 0.86f, -1.0f, 0.0f},
-    {14, 128, 128, 256, 0, 2.5f, 1.3f, 0.9f, 0.9f, -1.0f, 0.0f},
-    {11, 128, 64, 256, 0, 2.75f, 0.15f, 0.52f, 0.52f, -1.0f, 0.0f},
-    {35, 128, 80, 256, 0, 2.4f, 0.75f, 0.49f, 0.49f, -1.0f, 0.0f},
-    {40, 128, 128, 512, 0, 2.0f, 2.5f, 1.35f, 1.35f, -1.0f, 0.0f},
+    {41, 256, 160, 256, 0, 8.75f, 0.0f, 0.0f, 1.2f, 1.2f, -1.0f, 0.0f},
+    {24, 128, 160, 256, 0, 4.25f, 0.25f, 0.0f, 0.86f, 0.86f, -1.0f, 0.0f},
+    {14, 128, 128, 256, 0, 2.5f, 1.3f, 0.0f, 0.9f, 0.9f, -1.0f, 0.0f},
+    {11, 128, 64, 256, 0, 2.75f, 0.15f, 0.0f, 0.52f, 0.52f, -1.0f, 0.0f},
+    {35, 128, 80, 256, 0, 2.4f, 0.75f, 0.0f, 0.49f, 0.49f, -1.0f, 0.0f},
+    {40, 128, 128, 512, 0, 2.0f, 2.5f, 0.0f, 1.35f, 1.35f, -1.0f, 0.0f},
 };
 constexpr int kMaxSplits = 12;
 struct GemmPlan {
@@ -2042,7 +2044,7 @@ static GemmPlan plan_gemm(const TileCost (&tiles)[NT], int M, int N, int nk, boo
       // a last round with one workgroup to a CU instead of two runs faster
       float rounds = (float)ceil_div(grid * S, t.slots);
       if (t.slots == 512 && grid % 512 >= 1 && grid % 512 <= 256) rounds -= 0.4f;
-      const float fix = t.fix + (geglu ? t.geglu : 0.0f);
+      const float fix = t.fix + (geglu ? t.geglu : 0.0f) + (conv ? t.conv : 0.0f);
       const float us = rounds * (fix + (float)kps * (conv ? t.per_slice_conv : t.per_slice)) +
                        (S > 1 ? t.split0 + (float)S * t.split1 : 0.0f);
       if (us < best_t) {
