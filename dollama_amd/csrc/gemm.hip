@@ -2056,6 +2056,31 @@ static GemmPlan plan_gemm(const TileCost (&tiles)[NT], int M, int N, int nk, boo
   return best;
 }
 
+// Grids that the model above does not decide (0: it does).  `splits`: a split
+// of K is to be had.
+// Few outputs and a short K, where a split's exchange costs more than it saves
+// and a 128-row tile is mostly fill time: 64x16 tiles (43), up to two to a CU
+// (one where the rows are no whole 128-byte lines).  120 linears and 62 convs,
+// us: linear 1x216x8 3.1 on the register kernel, 4.4 on 128x64, 3.0 here;
+// 176x1280x1280 9.9 / 10.4 / 7.2; 300x1280x2560 15.6 / 14.4 / 12.8; conv
+// 8x488x576 8.5 / 10.0 / 6.8.  Past these lines the split 128x64 tiles are as
+// fast; where there are no splits, 64x16 stays faster at any K (300x1280x5120
+// 26.6 / 29.7 / 22.9).
+// Linears of half to one 64x64 tile per CU and a middling K: the
+// register-staged kernel (3) (1280x640x2560 15.9 us against 17.3 on split
+// 128x64 tiles, 828x640x2560 15.7 / 17.7; rows off the 128-byte lines cost the
+// DMA core 20% and it nothing: 2089x260x2384 15.4 / 20.4).  From 57 slices on
+// the splits are faster (1300x640x4096 22.8 / 20.8), below 20 the DMA tiles.
+// Without splits it stays ahead of the DMA tiles from there on too, for convs
+// as well (648x1280x11520 92 / 104 us).  It writes no GroupNorm statistics.
+static int small_grid_tile(int M, int N, int nk, bool conv, bool lines, bool gn, bool splits) {
+  constexpr int kCUs = 256;
+  if (ceil_div(M, 64) * ceil_div(N, 16) <= (lines ? 2 * kCUs : kCUs) && (!splits || nk <= (conv ? 28 : 40))) return 43;
+  const long long t64 = ceil_div(M, 64) * ceil_div(N, 64);
+  if (gn || t64 > kCUs || nk < 20) return 0;
+  return !splits || (!conv && t64 > kCUs / 2 && nk <= 56) ? 3 : 0;
+}
+
 static bool al8(const void* p) { return ((uintptr_t)p & 7) == 0; }
 
 // The DMA core needs 16-byte aligned operands (true of every RowDesc/ConvDesc
@@ -2202,31 +2227,22 @@ static int launch_gemm_impl(const Desc& ad, const RowDesc& bd, const EpiArgs& ep
         return launch_dma<192, 160, 48, 80, 3>(ad, bd, ep, M, N, s);
       constexpr bool conv = std::is_same<Desc, ConvDesc>::value;
       const int nk = (int)ceil_div(bd.K, BK);
-      if (!ep.vt && ep.act != DLM_ACT_GEGLU) {
-        // Few outputs and a short K, where a split's exchange costs more than
-        // it saves and a 128-row tile is mostly fill time: 64x16 tiles, up to
-        // two to a CU (one where the rows are no whole 128-byte lines).  120
-        // linears and 62 convs, us: linear 1x216x8 3.1 on the register
-        // kernel, 4.4 on 128x64, 2.9 here; 176x1280x1280 9.9 / 10.4 / 7.1;
-        // 300x1280x2560 15.6 / 14.4 / 12.8; conv 8x488x576 8.5 / 10.0 / 6.7.
-        // Past these lines the split 128x64 tiles are as fast.
-        const bool lines = (bd.ld | (conv ? 0 : bd.K)) % BK == 0;
-        if (ceil_div(M, 64) * ceil_div(N, 16) <= (lines ? 2 * kCUs : kCUs) && nk <= (conv ? 28 : 40))
-          return launch_dma<64, 16, 16, 16, 3>(ad, bd, ep, M, N, s);
-        // Linears of half to one 64x64 tile per CU and a middling K: the
-        // register-staged kernel (1280x640x2560 15.9 us against 17.3 on split
-        // 128x64 tiles, 828x640x2560 15.7 / 17.7; rows off the 128-byte lines
-        // cost the DMA core 20% and it nothing: 2089x260x2384 15.4 / 20.4).
-        // From 57 slices on the splits are faster (1300x640x4096 22.8 / 20.8),
-        // below 20 the DMA tiles.
-        const long long t64 = ceil_div(M, 64) * ceil_div(N, 64);
-        if (!conv && !ep.gn_stats && t64 > kCUs / 2 && t64 <= kCUs && nk >= 20 && nk <= 56)
-          return launch_cfg<64, 64, 32, 32>(ad, bd, ep, M, N, s);
+      const bool geglu = ep.act == DLM_ACT_GEGLU;
+      const bool splits = !t_no_split && !(g_variant & 1);
+      const bool lines = (bd.ld | (conv ? 0 : bd.K)) % BK == 0;
+      int tile = ep.vt || geglu ? 0 : small_grid_tile(M, N, nk, conv, lines, ep.gn_stats != nullptr, splits);
+      GemmPlan pl{tile, 1};
+      if (!tile) {
+        pl = plan_gemm(kTiles, M, N, nk, conv, geglu, splits ? kMaxSplits : 1);
+        // no workspace (a stream that met capture first, memory): plan without splits
+        if (pl.splits > 1 && !split_workspace(s)) {
+          if (!ep.vt && !geglu) tile = small_grid_tile(M, N, nk, conv, lines, ep.gn_stats != nullptr, false);
+          pl = tile ? GemmPlan{tile, 1} : plan_gemm(kTiles, M, N, nk, conv, geglu, 1);
+        }
       }
-      GemmPlan pl = plan_gemm(kTiles, M, N, nk, conv, ep.act == DLM_ACT_GEGLU, t_no_split || (g_variant & 1) ? 1 : kMaxSplits);
-      // no workspace (a stream that met capture first, memory): plan without splits
-      if (pl.splits > 1 && !split_workspace(s)) pl = plan_gemm(kTiles, M, N, nk, conv, ep.act == DLM_ACT_GEGLU, 1);
       switch (pl.tile) {
+        case 3: return launch_cfg<64, 64, 32, 32>(ad, bd, ep, M, N, s);
+        case 43: return launch_dma<64, 16, 16, 16, 3>(ad, bd, ep, M, N, s);
         case 11: return launch_dma<128, 64, 64, 32, 4>(ad, bd, ep, M, N, s, pl.splits);
         case 14: return launch_dma<128, 128, 64, 32, 4>(ad, bd, ep, M, N, s, pl.splits);
         case 19: return launch_dma<256, 128, 64, 64, 3>(ad, bd, ep, M, N, s);

@@ -241,6 +241,29 @@ def test_conv_planned_splits(gpu, B, H, W, Ci, Co, stride, up):
     assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
 
 
+def test_planned_without_splits(gpu):
+    """Where no split is to be had (a stream that met capture first), small grids with a long K take
+    the 64 x 16 tiles or the register-staged kernel: linears and convs on both sides of the lines."""
+    from dollama_amd import _lib
+    try:
+        _lib.call("dlm_gemm_set_variant", 1)
+        for M, N, K in ((300, 1280, 5120), (520, 1272, 5128), (600, 1280, 5120), (300, 340, 72)):
+            announce(f"linear without splits {M}x{N}x{K}")
+            x, w, b, r = randn((M, K), 174), randn((N, K), 175, std=K ** -0.5), randn((N,), 176), randn((M, N), 177)
+            y = ops.linear(to_gpu(x), to_gpu(w), bias=to_gpu(b), residual=to_gpu(r))
+            ref = x @ w.t() + b + r
+            assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
+        for B, H, W, Ci, Co, up in ((1, 9, 18, 640, 1280, True), (2, 12, 12, 640, 640, False)):
+            announce(f"conv without splits {B}x{H}x{W} {Ci}-{Co} up{up}")
+            x, w, b = randn((B, Ci, H, W), 178), randn((Co, Ci, 3, 3), 179, std=(9 * Ci) ** -0.5), randn((Co,), 180)
+            y = ops.nhwc_to_nchw(ops.conv2d_nhwc(ops.nchw_to_nhwc(to_gpu(x)), ops.pack_conv_weight(to_gpu(w)), KH=3,
+                                                 KW=3, pad=1, bias=to_gpu(b), upsample=up))
+            ref = torch.nn.functional.conv2d(R.upsample_nearest2x(x) if up else x, w, b, padding=1)
+            assert float((from_gpu(y) - ref).norm() / ref.norm()) <= 5e-4
+    finally:
+        _lib.call("dlm_gemm_set_variant", 0)
+
+
 @pytest.mark.parametrize("B,S,N,col0,K,ld", [(2, 77, 2560, 1280, 256, 80), (3, 12, 320, 160, 64, 16),
                                              (1, 1024, 1920, 1280, 64, 1024), (2, 100, 300, 100, 72, 104),
                                              (2, 988, 640, 320, 128, 992), (1, 131, 512, 128, 64, 133)])
