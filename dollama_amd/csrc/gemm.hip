@@ -1044,22 +1044,29 @@ __device__ __forceinline__ void vt_tile_store(const f16 DLM_LDS* st, int m0, int
 // 154x2560x2048 21.2 -> 16.1 us and 154x166400x2048 207 -> 199 us against the
 // per-block form (19.4 and 215 us where a lane walked every group of the
 // samples it touched, which took 134 us instead of 36 for the LayerNorm-folded
-// QKV of 2 x 999 tokens).
+// QKV of 2 x 999 tokens).  That QKV of 2 x 414 to 2 x 3302 tokens runs within
+// 3% of the per-block form.
 template <int BM, int BN, int TS, int NT>
 __device__ __forceinline__ void vt_tile_store_any(const f16 DLM_LDS* st, int m0, int n0, const EpiArgs& ep, int tid) {
   static_assert(BM <= NT, "a lane for every group: each holds at least one row of the tile");
   const int tokens = ep.vt_tokens, rows = min(BM, ep.M - m0);
+  // a / b for a <= NT: the quotient lies at least 1 / (2b) from an integer, far
+  // more than the reciprocal's error (an emulated integer division each cost
+  // the tile 0.5 us)
+  auto quot = [](int a, float rcp_b) { return (int)(((float)a + 0.5f) * rcp_b); };
   const int s0 = m0 / tokens, t0 = m0 - s0 * tokens;
   const int g0 = t0 >> 2, n0g = ((min(tokens, t0 + rows) + 3) >> 2) - g0;  // groups of the first sample
   const int gps = (tokens + 3) >> 2;                                       // of a whole sample
-  const int more = max(0, rows - (tokens - t0)), whole = more / tokens;    // rows of later samples
+  const int more = max(0, rows - (tokens - t0));                           // rows of later samples
+  const int whole = quot(more, __builtin_amdgcn_rcpf((float)tokens));
   const int groups = n0g + whole * gps + ((more - whole * tokens + 3) >> 2);
-  const int cs = NT / groups, c0 = tid / groups;
+  const float rg = __builtin_amdgcn_rcpf((float)groups);
+  const int cs = quot(NT, rg), c0 = quot(tid, rg);
   if (c0 >= cs) return;
   int g = tid - c0 * groups, smp = s0, tok = (g0 + g) * 4;
   if (g >= n0g) {
     g -= n0g;
-    const int ds = g / gps;
+    const int ds = quot(g, __builtin_amdgcn_rcpf((float)gps));
     smp = s0 + 1 + ds;
     tok = (g - ds * gps) * 4;
   }
@@ -1079,15 +1086,28 @@ __device__ __forceinline__ void vt_tile_store_any(const f16 DLM_LDS* st, int m0,
     off[e] = real[e] && in[e] ? r + e : 0;
   }
   const bool all = in[0] && in[1] && in[2] && in[3];
+  const bool pairs = !(tokens & 1);  // uniform: rows and tokens pair up on dwords
   for (int c = c0; c < cols; c += cs, dst += step, src += cs * TS) {
     f16x4 v;
+    if (pairs) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const f16 x = src[off[e]];
-      v[e] = real[e] ? x : (f16)0.0f;
+      for (int e = 0; e < 4; e += 2) {
+        const f16x2 x = *reinterpret_cast<const f16x2 DLM_LDS*>(src + off[e]);
+        v[e] = real[e] ? x[0] : (f16)0.0f;
+        v[e + 1] = real[e] ? x[1] : (f16)0.0f;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f16 x = src[off[e]];
+        v[e] = real[e] ? x : (f16)0.0f;
+      }
     }
     if (all) {
       *reinterpret_cast<f16x4*>(dst) = v;
+    } else if (pairs) {
+      if (in[0]) *reinterpret_cast<f16x2*>(dst) = f16x2{v[0], v[1]};
+      if (in[2]) *reinterpret_cast<f16x2*>(dst + 2) = f16x2{v[2], v[3]};
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -2065,14 +2085,14 @@ static GemmPlan plan_gemm(const TileCost (&tiles)[NT], int M, int N, int nk, boo
 // 176x1280x1280 9.9 / 10.4 / 7.2; 300x1280x2560 15.6 / 14.4 / 12.8; conv
 // 8x488x576 8.5 / 10.0 / 6.8.  Past these lines the split 128x64 tiles are as
 // fast; where there are no splits, 64x16 stays faster at any K (300x1280x5120
-// 26.6 / 29.7 / 22.9).
+// 26.6 / 29.8 / 23.1).
 // Linears of half to one 64x64 tile per CU and a middling K: the
 // register-staged kernel (3) (1280x640x2560 15.9 us against 17.3 on split
 // 128x64 tiles, 828x640x2560 15.7 / 17.7; rows off the 128-byte lines cost the
 // DMA core 20% and it nothing: 2089x260x2384 15.4 / 20.4).  From 57 slices on
 // the splits are faster (1300x640x4096 22.8 / 20.8), below 20 the DMA tiles.
 // Without splits it stays ahead of the DMA tiles from there on too, for convs
-// as well (648x1280x11520 92 / 104 us).  It writes no GroupNorm statistics.
+// as well (648x1280x11520 94 / 102 us).  It writes no GroupNorm statistics.
 static int small_grid_tile(int M, int N, int nk, bool conv, bool lines, bool gn, bool splits) {
   constexpr int kCUs = 256;
   if (ceil_div(M, 64) * ceil_div(N, 16) <= (lines ? 2 * kCUs : kCUs) && (!splits || nk <= (conv ? 28 : 40))) return 43;
