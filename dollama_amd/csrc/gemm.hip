@@ -1242,7 +1242,7 @@ __device__ __forceinline__ void split_coords(int bid, int tiles_m, int tiles_n, 
 // GEGLU launches gain 0.35 ms over the prefetch schedule and 0.12 ms over the
 // plain one, but the power they take slows the launches around them by more:
 // with FF1 on the prefetch schedule the step measured 0.30-0.32 ms faster on
-// two boxes and 0.03 slower on a third, on the plain one 0.10-0.21 ms faster
+// two cards and 0.03 slower on a third, on the plain one 0.10-0.21 ms faster
 // on four.  Launches that run alone keep the ping-pong.  Smaller
 // tiles, whose read phases are longer than their MFMA phases, measured slower
 // with it (128x128: 29 -> 34 us at 2048x3840x1280).
@@ -2033,7 +2033,7 @@ constexpr TileCost kTiles[] = {
 // of 60-9500 rows at 640 and 1280 channels, and GEGLU down to one K slice; the
 // choice is the fastest of the six everywhere, within 1%.  A fit to grids of
 // more than 256 tiles alone ran 128x128x4 tiles where 40 is faster, also with
-// one workgroup to a CU (1020x3840x1280 QKV 25.7 -> 22.1 us, start 23.8).
+// one workgroup to a CU (1020x3840x1280 QKV 25.7 -> 22.1 us).
 constexpr TileCost kLnTiles[] = {
     {41, 256, 160, 256, 0, 8.75f, 0.0f, 0.0f, 1.2f, 1.2f, -1.0f, 0.0f},
     {24, 128, 160, 256, 0, 4.25f, 0.25f, 0.0f, 0.86f, 0.86f, -1.0f, 0.0f},
